@@ -302,6 +302,7 @@ static hipError_t grid_launch(const ExactArgs& a, hipStream_t st, int64_t* nblk_
 hipError_t launch_exact(int op, const ExactArgs& a, double* max_out, hipStream_t st) {
   hipError_t e = hipErrorInvalidValue;
   int64_t nblk = 0;
+  if (a.mmtab && exact_mm_has(op)) return launch_exact_mm(op, a, st);
   switch (op) {
     case EX_DIV: e = grid_launch<EX_DIV, 2>(a, st, &nblk); break;
     case EX_SV2: e = grid_launch<EX_SV2, 4>(a, st, &nblk); break;
@@ -340,6 +341,10 @@ hipError_t launch_exact(int op, const ExactArgs& a, double* max_out, hipStream_t
       // than one fifteen-input pass)
       ExactArgs v, w;
       exact_evisc_split(a, a.rout2, v, w);
+      if (a.mmtab) {
+        if ((e = launch_exact_mm(EX_EVISCV, v, st)) != hipSuccess) return e;
+        return launch_exact_mm(EX_GRADMOM, w, st);
+      }
       if ((e = grid_launch<EX_EVISCV, 6>(v, st, &nblk)) != hipSuccess) return e;
       if ((e = grid_launch<EX_GRADMOM, 9>(w, st, &nblk)) != hipSuccess) return e;
       const int nmc = (w.M + EXACT_MC - 1) / EXACT_MC;

@@ -68,6 +68,7 @@ struct ExactArgs {
   const double* ctab;   // cos(2 pi m j/N) at [m*nj + j], sin at [(M + m)*nj + j], zero for j > K
   const double* rtab;   // (c_m/N) cos(2 pi j m/N) at [j*MR + m], (2/N) sin at [(K+1 + j)*MR + m],
                         // c_0 = 1, c_m = 2; zero for m >= M and for the sine of m = 0
+  const double* mmtab;  // tables of the matrix-core kernel (sfx_exact_mm_body.h), or null: two-pass kernels
   int nin, nout;
   ExactField in[EXACT_MAX_IN];
   ExactOut out[EXACT_MAX_OUT];

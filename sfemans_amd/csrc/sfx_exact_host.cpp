@@ -22,7 +22,10 @@ namespace sfx {
 static std::mutex g_exact_mu;
 static std::map<std::tuple<int, int, int>, double*> g_exact_tabs;
 
-static int exact_tables(int M, int K, const double** ctab, const double** rtab) {
+// the matrix-core tables, read two doubles at a time, start at an even offset
+static size_t exact_tables_even(size_t n) { return (n + 1) / 2 * 2; }
+
+static int exact_tables(int M, int K, const double** ctab, const double** rtab, const double** mmtab) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
@@ -31,17 +34,21 @@ static int exact_tables(int M, int K, const double** ctab, const double** rtab) 
   auto key = std::make_tuple(dev, M, K);
   auto it = g_exact_tabs.find(key);
   if (it == g_exact_tabs.end()) {
-    std::vector<double> h;
+    std::vector<double> h, mm;
     exact_host_tables(M, K, h);
+    if (exact_mm_sizes(M, K)) exact_mm_host_tables(M, K, h.data(), mm);
+    h.resize(exact_tables_even(nc + nr), 0.0);
+    h.insert(h.end(), mm.begin(), mm.end());
     double* d = nullptr;
-    e = hipMalloc(&d, (nc + nr) * sizeof(double));
+    e = hipMalloc(&d, h.size() * sizeof(double));
     if (e != hipSuccess) return fail(SFX_ERR_NOMEM, "hipMalloc(exact tables): %s", hipGetErrorString(e));
-    e = hipMemcpy(d, h.data(), (nc + nr) * sizeof(double), hipMemcpyHostToDevice);
+    e = hipMemcpy(d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "hipMemcpy(exact tables)");
     it = g_exact_tabs.emplace(key, d).first;
   }
   *ctab = it->second;
   *rtab = it->second + nc;
+  *mmtab = exact_mm_sizes(M, K) ? it->second + exact_tables_even(nc + nr) : nullptr;
   return SFX_OK;
 }
 
@@ -59,8 +66,11 @@ static int exact_prepare(const char* nm, ExactArgs& a, int op, int64_t np, int M
   if (m_max_pad < M) return fail(SFX_ERR_ARG, "%s: m_max_pad=%d < m_max=%d", nm, m_max_pad, M);
   if (m_max_pad > 4096) return fail(SFX_ERR_UNSUPPORTED, "%s: m_max_pad=%d > 4096", nm, m_max_pad);
   exact_setup_sizes(a, np, M, m_max_pad);
-  int rc = exact_tables(M, a.K, &a.ctab, &a.rtab);
+  int rc = exact_tables(M, a.K, &a.ctab, &a.rtab, &a.mmtab);
   if (rc) return rc;
+  // EX_EVISC's products are those of EX_GRADMOM on its last nine inputs
+  if (!exact_mm_use(op == EX_EVISC ? EX_GRADMOM : op, a)) a.mmtab = nullptr;
+  if (a.mmtab) return SFX_OK;   // no scratch
   void* w = nullptr;
   if (exact_is_reduction(op)) {
     const int64_t nb = exact_grid_blocks(op, a.nin, np, a.K);
@@ -183,7 +193,7 @@ static int emom_dev(const double* V1, const double* V2, const double* V3, const 
   ExactArgs a;
   exact_setup_emom(a, V1, V2, V3, c, hloc, out1, out2, np, M, lg, c2, c4);
   exact_setup_sizes(a, np, M, mp);
-  int rc = exact_tables(M, a.K, &a.ctab, &a.rtab);
+  int rc = exact_tables(M, a.K, &a.ctab, &a.rtab, &a.mmtab);
   if (rc) return rc;
   const int64_t ne = (np / lg) * (2 * (int64_t)mp - 1);
   void *w = nullptr, *pm = nullptr, *dm = nullptr;

@@ -6,7 +6,7 @@
 
 #include <vector>
 
-#include "sfx_exact_body.h"
+#include "sfx_exact_mm_body.h"
 
 namespace sfx {
 
@@ -30,6 +30,73 @@ inline void exact_host_tables(int M, int K, std::vector<double>& h) {
       h[nc + (size_t)j * MR + m] = (double)((m == 0 ? 1.0L : 2.0L) / (long double)N * c);
       h[nc + (size_t)(K + 1 + j) * MR + m] = m == 0 ? 0.0 : (double)(2.0L / (long double)N * s);
     }
+}
+
+// Whether the matrix-core kernel takes these sizes: accumulators for at most
+// two halves of 64 modes, and tables that stay in every L2.
+inline bool exact_mm_sizes(int M, int K) { return M >= 1 && M <= EXACT_MM_MAX_M && K + 1 <= EXACT_MM_MAX_PAD; }
+
+// Its tables (ExactMmArgs: ct then rt), from the ones of exact_host_tables.
+inline void exact_mm_host_tables(int M, int K, const double* h, std::vector<double>& t) {
+  const int nj = exact_nj(K), MR = exact_mr(M), MBN = exact_mm_mbn(M), JBN = exact_mm_jbn(K);
+  const double* r = h + exact_ctab_size(M, K);
+  const size_t nc = exact_mm_ctab_size(M, K);
+  t.assign(nc + exact_mm_rtab_size(M, K), 0.0);
+  for (int kb = 0; kb < 4 * MBN; ++kb)
+    for (int jb = 0; jb < JBN; ++jb)
+      for (int l = 0; l < 64; ++l) {
+        const int j = 16 * jb + l % 16, m = 4 * kb + l / 16;
+        if (j > K || m >= M) continue;
+        double* d = &t[((size_t)(kb * JBN + jb) * 64 + l) * 2];
+        d[0] = h[(size_t)m * nj + j];
+        d[1] = h[(size_t)(M + m) * nj + j];
+      }
+  for (int q = 0; q < 4 * JBN; ++q)
+    for (int mb = 0; mb < MBN; ++mb)
+      for (int l = 0; l < 64; ++l) {
+        const int m = 16 * mb + l % 16, j = 4 * q + l / 16;
+        if (j > K || m >= M) continue;
+        double* d = &t[nc + ((size_t)(q * MBN + mb) * 64 + l) * 2];
+        d[0] = r[(size_t)j * MR + m];
+        d[1] = r[(size_t)(K + 1 + j) * MR + m];
+      }
+}
+
+// The matrix-core kernel reads an input while other work-groups have already
+// stored outputs, so it does not take calls whose outputs overlap inputs (the
+// two-pass kernels read everything before the first store).
+inline bool exact_mm_disjoint(const ExactArgs& a) {
+  for (int g = 0; g < a.nout; ++g) {
+    const ExactOut& o = a.out[g];
+    const double *o0 = o.base, *o1 = o.base + (a.np - 1) * o.sp + (a.M - 1) * o.sm + o.off + 1;
+    for (int f = 0; f < a.nin; ++f) {
+      const ExactField& i = a.in[f];
+      if (!i.base) continue;
+      if (o0 < i.base + (a.np - 1) * i.sp + (a.M - 1) * i.sm + i.off + 1 && i.base < o1) return false;
+    }
+    if (a.creal && o0 < a.creal + a.n_creal && a.creal < o1) return false;
+  }
+  return true;
+}
+
+// Whether a product runs on the matrix-core kernel.  Times, two-pass kernels /
+// matrix-core kernel in us, on 60,000 points unless said otherwise:
+// - its exact form (M <= 64 on a grid of 3/2 as many angle pairs) is faster at
+//   every number of points: v / s 154 / 76 at M = 32, 464 / 236 at M = 64 and
+//   59 / 19 on 500 points, tension tensor 1101 / 767 at M = 64;
+// - but blocks of 16 modes are mostly empty for a few modes: v / s 19 / 20 and
+//   tension 37 / 75 at M = 4, tension 65 / 78 and v / s 30 / 22 at M = 8;
+// - the general form repeats the synthesis for the second half of the modes:
+//   v / s 662 / 707 at M = 80 and 1148 / 1305 at M = 112, but on 500 points,
+//   where the two-pass kernels leave the chip idle, 81 / 30 and 146 / 49;
+// - the analysis alone (EX_FROMREAL) has no synthesis: 238 / 87 at M = 80.
+inline bool exact_mm_use(int op, const ExactArgs& a) {
+  if (!exact_mm_has(op) || a.np <= 0 || !exact_mm_sizes(a.M, a.K) || !exact_mm_disjoint(a)) return false;
+  if (op == EX_FROMREAL) return true;
+  const int jb = exact_mm_jb(exact_mm_mb(a.M)), jbn = exact_mm_jbn(a.K);
+  if (a.M > 64 || (jbn != jb && jbn != jb - 1)) return a.np <= 2048;
+  const bool few = a.M <= 4 || (a.M <= 8 && (op == EX_TENSION || op == EX_COMPR));
+  return !few || a.np <= 16384;
 }
 
 inline void exact_setup_sizes(ExactArgs& a, int64_t np, int M, int m_max_pad) {

@@ -84,6 +84,8 @@ hipError_t launch_gauss(int variant, const GaussArgs& a, hipStream_t st);
 hipError_t launch_fftprod(int op, const FftProdArgs& a, hipStream_t st);
 // Exact-grid products (sfx_exact_body.h): angle pass, then r2c, or the maximum into max_out.
 struct ExactArgs;
+// The same on the matrix cores (a.mmtab set, sfx_exact_mm_body.h).
+hipError_t launch_exact_mm(int op, const ExactArgs& a, hipStream_t st);
 hipError_t launch_exact(int op, const ExactArgs& a, double* max_out, hipStream_t st);
 hipError_t launch_exact_velstat(const ExactArgs& a, double* part, double* out, hipStream_t st);
 int64_t exact_velstat_blocks(int nin, int64_t np, int K);

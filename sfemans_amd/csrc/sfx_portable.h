@@ -19,6 +19,14 @@ void sfx_emu_sync();
 void sfx_emu_wave_sync();
 [[noreturn]] void sfx_emu_oob(const char* what, long long idx, long long n, const char* file, int line);
 #define SFX_SYNC() sfx_emu_sync()
+struct sfx_d4 {
+  double v[4];
+  double& operator[](int i) { return v[i]; }
+  const double& operator[](int i) const { return v[i]; }
+};
+sfx_d4 sfx_emu_mfma_f64(double a, double b, const sfx_d4& c);
+#define SFX_MFMA_F64(a, b, c) sfx_emu_mfma_f64((a), (b), (c))
+#define SFX_UNIFORM(x) (x)
 #define SFX_WAVE_SYNC() sfx_emu_wave_sync()
 #define SFX_OPAQUE(x) do { } while (0)
 #define SFX_OPAQUE_S(x) do { } while (0)
@@ -41,6 +49,13 @@ void sfx_emu_wave_sync();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); \
   } while (0)
 #define SFX_CHECK(what, idx, n) do { } while (0)
+// c + a b on the matrix core: a 16x4 (lane l holds row l % 16, column l / 16),
+// b 4x16 (row l / 16, column l % 16), c 16x16 (element v of lane l: row l / 16
+// + 4 v, column l % 16).
+typedef double sfx_d4 __attribute__((ext_vector_type(4)));
+#define SFX_MFMA_F64(a, b, c) __builtin_amdgcn_mfma_f64_16x16x4f64((a), (b), (c), 0, 0, 0)
+// An int that is the same in every lane of the wave, as a scalar.
+#define SFX_UNIFORM(x) __builtin_amdgcn_readfirstlane(x)
 // Hide a value's origin from the optimizer, so that what is computed from it
 // is recomputed where it is used instead of being kept live (or spilled)
 // across a long stretch of code.  Emits no instruction.

@@ -22,8 +22,22 @@
 
 static thread_local std::barrier<>* g_bar = nullptr;        // work-group barrier
 static thread_local std::barrier<>* g_wave_bar = nullptr;   // barrier of the thread's wave (64 threads)
+static thread_local double (*g_wave_ab)[64] = nullptr;       // the wave's matrix-core operands a, b
+static thread_local int g_lane = 0;
 void sfx_emu_sync() { g_bar->arrive_and_wait(); }
 void sfx_emu_wave_sync() { g_wave_bar->arrive_and_wait(); }
+// v_mfma_f64_16x16x4: every lane of the wave calls it together
+sfx_d4 sfx_emu_mfma_f64(double a, double b, const sfx_d4& c) {
+  g_wave_ab[0][g_lane] = a;
+  g_wave_ab[1][g_lane] = b;
+  g_wave_bar->arrive_and_wait();
+  sfx_d4 d = c;
+  for (int v = 0; v < 4; ++v)
+    for (int k = 0; k < 4; ++k)
+      d[v] = std::fma(g_wave_ab[0][16 * k + g_lane / 16 + 4 * v], g_wave_ab[1][16 * k + g_lane % 16], d[v]);
+  g_wave_bar->arrive_and_wait();
+  return d;
+}
 void sfx_emu_oob(const char* what, long long idx, long long n, const char* file, int line) {
   std::fprintf(stderr, "SFX_EMU out of bounds: %s index %lld not in [0,%lld) at %s:%d\n", what, idx, n, file, line);
   std::fflush(stderr);
@@ -43,11 +57,13 @@ static void run_grid(int64_t nblk, int threads, size_t smem_cplx,
     std::vector<std::unique_ptr<std::barrier<>>> wbar;
     for (int w = 0; w < (threads + 63) / 64; ++w)
       wbar.emplace_back(new std::barrier<>(std::min(64, threads - 64 * w)));
+    std::vector<double> ab((size_t)wbar.size() * 128);
     for (auto& x : smem) x = make_double2(1e300, -1e300);   // poison: stale reads show up
     std::vector<std::thread> th;
     th.reserve(threads);
     for (int t = 0; t < threads; ++t)
-      th.emplace_back([&, t] { g_bar = &bar; g_wave_bar = wbar[t / 64].get(); body(t, b, smem.data()); });
+      th.emplace_back([&, t] { g_bar = &bar; g_wave_bar = wbar[t / 64].get();
+                            g_wave_ab = reinterpret_cast<double(*)[64]>(&ab[(size_t)(t / 64) * 128]); g_lane = t % 64; body(t, b, smem.data()); });
     for (auto& x : th) x.join();
     for (size_t i = smem_cplx; i < smem.size(); ++i)
       if (smem[i].x != 1e300 || smem[i].y != -1e300) sfx_emu_oob("LDS guard", (long long)i, (long long)smem_cplx, __FILE__, __LINE__);
@@ -450,8 +466,9 @@ static void emu_exact_grid(const ExactArgs& a, double& vmax) {
 // FFT_COMPUTE_ENTROPY_VISC: V = [V1 .. V5] (5 x np*6*M), out = [O1 | O2 | O3];
 // the element maxima as exact_enorm_kernel computes them (32 elements and 16
 // angle pairs per work-group, one thread per point).
-extern "C" int emu_exact_evisc(int64_t np, int M, int mp, int lg, const double* V, const double* hloc, double c1,
-                               double c2, double c4, double res, double* out) {
+static int emu_exact_mm_op(int op, ExactArgs& a);
+static int emu_evisc(bool mm, int64_t np, int M, int mp, int lg, const double* V, const double* hloc, double c1,
+                     double c2, double c4, double res, double* out) {
   const int64_t n6 = np * 6 * M;
   const double* Vp[5] = {V, V + n6, V + 2 * n6, V + 3 * n6, V + 4 * n6};
   double* O[3] = {out, out + n6, out + 2 * n6};
@@ -500,12 +517,66 @@ extern "C" int emu_exact_evisc(int64_t np, int M, int mp, int lg, const double* 
   ExactArgs v, w;
   exact_evisc_split(a, vreal.data(), v, w);
   double vmax = 0.0;
+  if (mm) {
+    const int rc = emu_exact_mm_op(EX_EVISCV, v);
+    return rc ? rc : emu_exact_mm_op(EX_GRADMOM, w);
+  }
   emu_exact_grid<EX_EVISCV, 6>(v, vmax);
   emu_exact_grid<EX_GRADMOM, 9>(w, vmax);
   const int nmc = (M + EXACT_MC - 1) / EXACT_MC;
   for (int64_t p = 0; p < np; ++p)
     for (int g = 0; g < w.nout; ++g)
       for (int mc = 0; mc < nmc; ++mc) exact_r2c_body(w, p, g, mc);
+  return 0;
+}
+
+extern "C" int emu_exact_evisc(int64_t np, int M, int mp, int lg, const double* V, const double* hloc, double c1,
+                               double c2, double c4, double res, double* out) {
+  return emu_evisc(false, np, M, mp, lg, V, hloc, c1, c2, c4, res, out);
+}
+extern "C" int emu_exact_evisc_mm(int64_t np, int M, int mp, int lg, const double* V, const double* hloc, double c1,
+                                  double c2, double c4, double res, double* out) {
+  return emu_evisc(true, np, M, mp, lg, V, hloc, c1, c2, c4, res, out);
+}
+
+extern "C" int emu_exact(int op, int64_t np, int M, int mp, const double* in1, const double* in2,
+                         const double* values, int n_values, double eps, int nb, double* out);
+
+// The argument sets of emu_exact (below); cls_vmax holds EX_CLS's velocity maximum.
+static int emu_exact_setup(ExactArgs& a, double& cls_vmax, int op, int64_t np, int M, int mp, const double* in1,
+                           const double* in2, const double* values, int n_values, double eps, int nb, double* out) {
+  switch (op) {
+    case EX_DIV: exact_setup_div(a, in1, in2, out, np, M); break;
+    case EX_SV2: exact_setup_sv2(a, in1, in2, out, np, M); break;
+    case EX_SQRT: exact_setup_sqrt(a, in1, out, np, nb, M); break;
+    case EX_HEAVI: exact_setup_heavi(a, in1, values, n_values, out, np, M, eps); break;
+    case EX_TENSION: exact_setup_tension(a, in1, in2, out, np, M); break;
+    case EX_MAXVEL: exact_setup_maxvel(a, in1, np, nb, M); break;
+    case EX_SVCLAMP: exact_setup_svclamp(a, in1, in2, out, np, M, nb, values[0], values[1]); break;
+    case EX_CLAMP01: exact_setup_sqrt(a, in1, out, np, nb, M); break;
+    case EX_ENTRO:   // in2 = c (np,2,M) then c_in_real (N,np) packed after it; out = V_out then c_out
+      exact_setup_entro(a, in1, in2, in2 + 2 * np * M, values[0], out, out + 6 * np * M, np, M, mp);
+      break;
+    case EX_GRADMOM:   // in1 = [V1 | V2 | V3] (3 x np*6*M) then c_in_real (N, np); values = {coeff}
+      exact_setup_gradmom(a, in1, in1 + 6 * np * M, in1 + 12 * np * M, in1 + 18 * np * M, values[0], out, np, M, mp);
+      break;
+    case EX_COMPR:   // in1 = [V1 | V2] (2 x np*6*M), in2 = [c (np,2,M) | c_in_real (N,np)],
+                     // values = {coeff, comp}, out = [V_out | c_out]
+      exact_setup_compr(a, in1, in1 + 6 * np * M, in2, in2 + 2 * np * M, values[0], values[1], out,
+                        out + 6 * np * M, np, M, mp);
+      break;
+    case EX_CLS: {   // in1 = [grad phi | velocity] (2 x np*6*M), in2 = phi (np,2,M),
+                     // values = {level_set_comp_factor, LES_coeff4, h_min_distance}
+      const int rc = emu_exact(EX_MAXVEL, np, M, mp, in1 + 6 * np * M, nullptr, nullptr, 0, 0.0, 6, &cls_vmax);
+      if (rc) return rc;
+      exact_setup_cls(a, in1, in2, out, &cls_vmax, np, M, values[0], values[1], values[2]);
+      break;
+    }
+    case EX_ETA:     // 17/18 eta products: in1 = c (np, nb, M), in2 = eta (N, np)
+    case EX_ETA3: exact_setup_eta(a, in2, in1, out, np, nb, M, mp); break;
+    case EX_FROMREAL: exact_setup_fromreal(a, in2, out, np, M, mp); break;   // 19: in2 = values (N, np)
+    default: return 1;
+  }
   return 0;
 }
 
@@ -568,38 +639,7 @@ extern "C" int emu_exact(int op, int64_t np, int M, int mp, const double* in1, c
     }
     return 0;
   }
-  switch (op) {
-    case EX_DIV: exact_setup_div(a, in1, in2, out, np, M); break;
-    case EX_SV2: exact_setup_sv2(a, in1, in2, out, np, M); break;
-    case EX_SQRT: exact_setup_sqrt(a, in1, out, np, nb, M); break;
-    case EX_HEAVI: exact_setup_heavi(a, in1, values, n_values, out, np, M, eps); break;
-    case EX_TENSION: exact_setup_tension(a, in1, in2, out, np, M); break;
-    case EX_MAXVEL: exact_setup_maxvel(a, in1, np, nb, M); break;
-    case EX_SVCLAMP: exact_setup_svclamp(a, in1, in2, out, np, M, nb, values[0], values[1]); break;
-    case EX_CLAMP01: exact_setup_sqrt(a, in1, out, np, nb, M); break;
-    case EX_ENTRO:   // in2 = c (np,2,M) then c_in_real (N,np) packed after it; out = V_out then c_out
-      exact_setup_entro(a, in1, in2, in2 + 2 * np * M, values[0], out, out + 6 * np * M, np, M, mp);
-      break;
-    case EX_GRADMOM:   // in1 = [V1 | V2 | V3] (3 x np*6*M) then c_in_real (N, np); values = {coeff}
-      exact_setup_gradmom(a, in1, in1 + 6 * np * M, in1 + 12 * np * M, in1 + 18 * np * M, values[0], out, np, M, mp);
-      break;
-    case EX_COMPR:   // in1 = [V1 | V2] (2 x np*6*M), in2 = [c (np,2,M) | c_in_real (N,np)],
-                     // values = {coeff, comp}, out = [V_out | c_out]
-      exact_setup_compr(a, in1, in1 + 6 * np * M, in2, in2 + 2 * np * M, values[0], values[1], out,
-                        out + 6 * np * M, np, M, mp);
-      break;
-    case EX_CLS: {   // in1 = [grad phi | velocity] (2 x np*6*M), in2 = phi (np,2,M),
-                     // values = {level_set_comp_factor, LES_coeff4, h_min_distance}
-      const int rc = emu_exact(EX_MAXVEL, np, M, mp, in1 + 6 * np * M, nullptr, nullptr, 0, 0.0, 6, &cls_vmax);
-      if (rc) return rc;
-      exact_setup_cls(a, in1, in2, out, &cls_vmax, np, M, values[0], values[1], values[2]);
-      break;
-    }
-    case EX_ETA:     // 17/18 eta products: in1 = c (np, nb, M), in2 = eta (N, np)
-    case EX_ETA3: exact_setup_eta(a, in2, in1, out, np, nb, M, mp); break;
-    case EX_FROMREAL: exact_setup_fromreal(a, in2, out, np, M, mp); break;   // 19: in2 = values (N, np)
-    default: return 1;
-  }
+  if (const int rc = emu_exact_setup(a, cls_vmax, op, np, M, mp, in1, in2, values, n_values, eps, nb, out)) return rc;
   exact_setup_sizes(a, np, M, mp);
   std::vector<double> tab;
   exact_host_tables(M, a.K, tab);
@@ -641,6 +681,76 @@ extern "C" int emu_exact(int op, int64_t np, int M, int mp, const double* in1, c
     for (int g = 0; g < a.nout; ++g)
       for (int mc = 0; mc < nmc; ++mc) exact_r2c_body(a, p, g, mc);
   return 0;
+}
+
+// The same products on the matrix-core kernel (sfx_exact_mm_body.h).
+template <int OP, int NIN, int MB>
+static void emu_exact_mm_run(const ExactMmArgs& A) {
+  constexpr int NI = exact_mm_nin(OP, NIN), NO = exact_mm_nout(OP);
+  for (int y = 0; y < exact_mm_groups(OP); ++y)
+    for (int z = 0; z < (NO > 0 ? (A.mbn + MB - 1) / MB : 1); ++z)
+      run_grid((A.a.np + 15) / 16, 64 * exact_mm_waves(NI, NO), exact_mm_smem(NI) / 2,
+               [&](int t, int64_t b, double2* sm) {
+                 double* d = reinterpret_cast<double*>(sm);
+                 constexpr int JB = exact_mm_jb(MB);   // as the GPU launcher
+                 if (A.mbn == MB && A.jbn == JB) exact_mm_body<OP, NIN, MB, JB, true>(A, t, b, y, z, d);
+                 else if (A.mbn == MB && A.jbn == JB - 1) exact_mm_body<OP, NIN, MB, JB - 1, true>(A, t, b, y, z, d);
+                 else exact_mm_body<OP, NIN, MB, JB, false>(A, t, b, y, z, d);
+               });
+}
+template <int OP, int NIN>
+static int emu_exact_mm_m(const ExactMmArgs& A) {
+  switch (exact_mm_mb(A.a.M)) {
+    case 1: emu_exact_mm_run<OP, NIN, 1>(A); return 0;
+    case 2: emu_exact_mm_run<OP, NIN, 2>(A); return 0;
+    case 3: emu_exact_mm_run<OP, NIN, 3>(A); return 0;
+    case 4: emu_exact_mm_run<OP, NIN, 4>(A); return 0;
+    }
+    return 2;
+}
+static int emu_exact_mm_op(int op, ExactArgs& a) {
+  std::vector<double> tab, mm;
+  exact_host_tables(a.M, a.K, tab);
+  if (!exact_mm_sizes(a.M, a.K) || !exact_mm_disjoint(a)) return 4;
+  exact_mm_host_tables(a.M, a.K, tab.data(), mm);
+  ExactMmArgs A;
+  A.a = a;
+  A.mbn = exact_mm_mbn(a.M); A.jbn = exact_mm_jbn(a.K);
+  A.n_ct = (int64_t)exact_mm_ctab_size(a.M, a.K); A.n_rt = (int64_t)exact_mm_rtab_size(a.M, a.K);
+  A.ct = mm.data(); A.rt = mm.data() + A.n_ct;
+  switch (op) {   // as launch_exact_mm
+    case EX_DIV: return emu_exact_mm_m<EX_DIV, 2>(A);
+    case EX_SV2: return emu_exact_mm_m<EX_SV2, 4>(A);
+    case EX_SVCLAMP: return emu_exact_mm_m<EX_SVCLAMP, 4>(A);
+    case EX_SQRT: return emu_exact_mm_m<EX_SQRT, 1>(A);
+    case EX_CLAMP01: return emu_exact_mm_m<EX_CLAMP01, 1>(A);
+    case EX_TENSION: return emu_exact_mm_m<MM_TENSROW, 4>(A);
+    case EX_ENTRO: return emu_exact_mm_m<EX_ENTRO, 4>(A);
+    case EX_GRADMOM: return emu_exact_mm_m<MM_SCALE3, 3>(A);
+    case EX_COMPR: return emu_exact_mm_m<EX_COMPR, 7>(A);
+    case EX_CLS: return emu_exact_mm_m<EX_CLS, 4>(A);
+    case EX_ETA: return emu_exact_mm_m<EX_ETA, 1>(A);
+    case EX_ETA3: return emu_exact_mm_m<EX_ETA3, 3>(A);
+    case EX_FROMREAL: return emu_exact_mm_m<EX_FROMREAL, 0>(A);
+    case EX_EVISCV: return emu_exact_mm_m<EX_EVISCV, 6>(A);
+    case EX_HEAVI:
+      return a.nin == 1 ? emu_exact_mm_m<EX_HEAVI, 1>(A) : a.nin == 2 ? emu_exact_mm_m<EX_HEAVI, 2>(A)
+             : a.nin == 3 ? emu_exact_mm_m<EX_HEAVI, 3>(A) : emu_exact_mm_m<EX_HEAVI, 4>(A);
+  }
+  return 1;
+}
+extern "C" int emu_exact_mm(int op, int64_t np, int M, int mp, const double* in1, const double* in2,
+                            const double* values, int n_values, double eps, int nb, double* out) {
+  ExactArgs a;
+  double cls_vmax = 0.0;
+  std::vector<double> copy;
+  if (op == EX_SQRT || op == EX_CLAMP01) {   // in place: the library passes a copy
+    copy.assign(in1, in1 + np * nb * M);
+    in1 = copy.data();
+  }
+  if (const int rc = emu_exact_setup(a, cls_vmax, op, np, M, mp, in1, in2, values, n_values, eps, nb, out)) return rc;
+  exact_setup_sizes(a, np, M, mp);
+  return emu_exact_mm_op(op, a);
 }
 
 // FFT_COMPUTE_ENTROPY_VISC_MOM: V = [V1 | V2 | V3] (3 x np*6*M), c (np,2,M),

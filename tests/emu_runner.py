@@ -73,8 +73,12 @@ def _load(path: str = LIB):
     L.emu_batch.restype = C.c_int
     L.emu_exact.argtypes = [i32, i64, i32, i32, vp, vp, vp, i32, C.c_double, i32, vp]
     L.emu_exact.restype = C.c_int
+    L.emu_exact_mm.argtypes = L.emu_exact.argtypes
+    L.emu_exact_mm.restype = C.c_int
     L.emu_exact_evisc.argtypes = [i64, i32, i32, i32, vp, vp, C.c_double, C.c_double, C.c_double, C.c_double, vp]
     L.emu_exact_evisc.restype = C.c_int
+    L.emu_exact_evisc_mm.argtypes = L.emu_exact_evisc.argtypes
+    L.emu_exact_evisc_mm.restype = C.c_int
     L.emu_exact_emom.argtypes = [i64, i32, i32, i32, vp, vp, vp, C.c_double, C.c_double, vp, vp]
     L.emu_exact_emom.restype = C.c_int
     L.emu_dotsf.argtypes = [vp, vp, i64, i64, vp, i32, i32, vp, vp, i64, vp]
