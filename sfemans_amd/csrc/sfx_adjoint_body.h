@@ -153,7 +153,7 @@ SFX_DEV void load_ybar(const AdjArgs& A, int64_t p, bool valid, int pt, int l, d
     // round A slots 0 and 3, round B slots 1 and 2.  The partner of slot r
     // is slot 3 - r at lane (L - l) % L for l >= 1, slot (4 - r) % 4 of
     // lane 0 for l = 0 (whose slot-0 partner, mode MP, is dropped by pack).
-    const int lane = pt * L + l, plane = pt * L + (L - l) % L;
+    const int lane = lane_at<MP>(pt, l), plane = lane_partner<MP>(pt, l);
     const bool l0 = (l == 0);
     double a0[6], a1[6], b0[6], b1[6];
 #pragma unroll
@@ -200,7 +200,7 @@ SFX_DEV void load_ybar(const AdjArgs& A, int64_t p, bool valid, int pt, int l, d
   } else {
     // mode MP - m of slot r is held by lane (L - l) % L in slot 3 - r (l >= 1)
     // or 4 - r (l = 0, r >= 1); layout xf[(6 slot + c) * 64 + lane]
-    const int lane = pt * L + l, plane = pt * L + (L - l) % L;
+    const int lane = lane_at<MP>(pt, l), plane = lane_partner<MP>(pt, l);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -241,7 +241,7 @@ SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem)
   constexpr int GX = AL::GX;
   constexpr int NT = 64 * NW;
   const int wave = tid >> 6, lane = tid & 63;
-  const int pt = lane / L, l = lane % L;
+  const int pt = lane_pt<MP>(lane), l = lane_l<MP>(lane);
   double* smd = reinterpret_cast<double*>(smem);
   double2* tw = smem + LY::TW;
   double* tab = smd + 2 * LY::TAB;

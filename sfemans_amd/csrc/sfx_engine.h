@@ -19,7 +19,7 @@
 // The length-MP transforms are radix-4 decimation-in-frequency stages (with a
 // final radix-2 stage when log2 MP is odd).  A point is handled by L = MP/4
 // lanes holding 4 values each, so a 64-lane wave carries PW = 256/MP points.
-// Between stages the values are exchanged through a wave-private LDS region.
+// Between stages the lanes of a point exchange their values (exchange below).
 // The forward transform applies the conjugate transposes of the inverse
 // stages in reverse order; it starts from the inverse's digit-reversed output
 // positions (a pointwise product commutes with that permutation) and ends
@@ -75,21 +75,36 @@ SFX_DEV int stage_pos(int s, int l, int r) {
   return 4 * l + r;
 }
 
+// Lane of a wave <-> (point pt, lane l of the point): the points are fastest,
+// so that the lanes that hold one mode of consecutive points are neighbours
+// and the two leading bits of l, which the first exchange transposes with the
+// value index, are the leading bits of the lane.
+template <int MP>
+SFX_DEV int lane_pt(int lane) { return lane % Shape<MP>::PW; }
+template <int MP>
+SFX_DEV int lane_l(int lane) { return lane / Shape<MP>::PW; }
+template <int MP>
+SFX_DEV int lane_at(int pt, int l) { return l * Shape<MP>::PW + pt; }
+// Lane of the same point that holds the partner modes MP - m of lane l.
+template <int MP>
+SFX_DEV int lane_partner(int pt, int l) { return lane_at<MP>(pt, (Shape<MP>::L - l) % Shape<MP>::L); }
+
 // LDS slot of (point, position) inside a wave region for exchange `ex`
 // (ex = s for the exchange between stages s and s+1, ex = 4 for the mode
 // pairing).  q = pt*MP + pos indexes the 256 slots of one signal; the low
 // four bits are XORed with a GF(2)-linear function of bits 2..7 of q.  The
 // per-exchange masks were found by exhaustive search so that every 8- and
-// 16-lane group of every access pattern hits distinct 16-byte bank groups;
-// masks on bits 2 and 3 only touch bits 0 and 1, so the map is a bijection.
+// 16-lane group of every access pattern hits distinct 16-byte bank groups
+// (8-lane groups at MP = 128, ex = 4: two-way); masks on bits 2 and 3 only
+// touch bits 0 and 1, so the map is a bijection.
 constexpr unsigned char SWZ[7][5][6] = {
-  {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}},  // MP=4
-  {{1,3,15,2,6,6}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {3,2,5,7,3,7}},  // MP=8
-  {{0,3,14,6,9,4}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {3,0,15,7,11,10}},  // MP=16
-  {{0,2,14,12,15,10}, {2,3,7,8,13,7}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {3,0,8,8,0,4}},  // MP=32
-  {{2,0,4,14,1,5}, {3,2,12,5,15,3}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,12,3}},  // MP=64
-  {{0,2,15,13,15,14}, {1,2,14,8,11,11}, {0,2,15,6,0,1}, {0,0,0,0,0,0}, {3,0,0,0,0,15}},  // MP=128
-  {{3,3,9,2,13,3}, {0,2,7,12,8,14}, {3,1,12,8,0,14}, {0,0,0,0,0,0}, {0,0,0,0,0,0}},  // MP=256
+  {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,1,2,1,0,0}},  // MP=4
+  {{0,1,4,2,1,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,1,4,2,1,0}},  // MP=8
+  {{0,0,9,4,2,1}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,9,4,2,1}},  // MP=16
+  {{0,0,0,9,4,2}, {1,0,0,9,4,2}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,1,0,9,4,2}},  // MP=32
+  {{0,0,0,0,10,4}, {1,0,0,0,10,4}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,2,0,0,10,4}},  // MP=64
+  {{0,0,0,0,0,12}, {0,2,2,0,0,12}, {1,2,2,0,0,4}, {0,0,0,0,0,0}, {0,0,0,0,0,8}},  // MP=128
+  {{0,0,0,0,0,0}, {0,0,12,4,0,0}, {2,1,12,4,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}},  // MP=256
 };
 
 template <int MP>
@@ -162,16 +177,72 @@ SFX_DEV void fwd_stage(int s, int l, double2 (&v)[4], const double2* __restrict_
   }
 }
 
-// Exchange a group of NS signals from stage layout `sa` to stage layout `sb`.
-// `lds` is this wave's region: NS * WAVE_CPLX complex slots.
+// Exchange s (between stages s and s + 1, either way) transposes the value
+// index with bits of l: between radix-4 stages the two bits of the index with
+// the two leading bits of l that stage s strides over; before the final
+// radix-2 stage one bit.  EXCH_BIT: the lane bit of the lower of them.
+template <int MP>
+constexpr int exch_bit(int s) {
+  // stage s strides over the lowest LOG2 - 2 s - 2 bits of l, l starts at lane bit log2(PW) = 8 - LOG2
+  const int low = (Shape<MP>::LOG2 - 2 * s - 2) - (s + 1 < Shape<MP>::N4 ? 2 : 1) + 8 - Shape<MP>::LOG2;
+  return 1 << low;
+}
+
+// Transpose the value index bit of (a, b) with lane bit BIT: a becomes the
+// pair's value from the lane whose bit is 0, b the one from the lane whose bit
+// is 1, each of the index that the own bit says.
+template <int BIT>
+SFX_DEV void lane_swap(double2& a, double2& b) {
+  SFX_LANE_SWAP(a.x, b.x, BIT);
+  SFX_LANE_SWAP(a.y, b.y, BIT);
+}
+
+// Exchange a group of NS signals from stage layout `sa` to stage layout `sb`
+// (neighbours).  Over lane bits 4 and 5 a pair of registers takes one
+// v_permlane*_swap per bit (8 cycles), over bits 2 and 3 two DPP moves and a
+// copy (12 cycles); over bits 0 and 1 (the last exchange at MP = 128 and 256) the
+// values go through `lds`, this wave's region of NS * WAVE_CPLX complex slots.
+// Through LDS the 4 values of a lane cost 283 cycles of the CU's LDS per wave on
+// each SIMD (a write moves 75 bytes per cycle, a 16-byte read 270) plus its
+// latency, against 133 (bits 4, 5) and 183 cycles of the SIMD's own vector
+// unit; the lanes of a point used to be consecutive, with every exchange in
+// LDS.  Both changes together at 200,704 triangles, M = 64: forward term 5.26
+// -> 4.23 ms, adjoint 10.50 -> 9.37 ms, cross product on 402,753 points 1.19 ->
+// 1.06 ms; with the exchange over bits 2 and 3 in LDS 4.58, 9.67 and 1.10 ms.
 template <int MP, int NS>
 SFX_DEV void exchange(double2 (*v)[4], int sa, int sb, int pt, int l, double2* lds) {
   constexpr int WC = Shape<MP>::WAVE_CPLX;
+  const int s = sa < sb ? sa : sb;
+  const bool r4 = s + 1 < Shape<MP>::N4;
+  const int bit = exch_bit<MP>(s);
+  if (bit >= 4) {
+#pragma unroll
+    for (int g = 0; g < NS; ++g) {
+      double2(&w)[4] = v[g];
+      // before the radix-2 stage, positions 4 l + 2 r0 + o: the value index is (r0, o)
+      if (!r4 && sa > sb) { const double2 t = w[1]; w[1] = w[2]; w[2] = t; }
+      if (r4) {
+        if (bit == 16) {
+          lane_swap<32>(w[0], w[2]); lane_swap<32>(w[1], w[3]);
+          lane_swap<16>(w[0], w[1]); lane_swap<16>(w[2], w[3]);
+        } else {
+          lane_swap<8>(w[0], w[2]); lane_swap<8>(w[1], w[3]);
+          lane_swap<4>(w[0], w[1]); lane_swap<4>(w[2], w[3]);
+        }
+      } else if (bit == 32) {
+        lane_swap<32>(w[0], w[2]); lane_swap<32>(w[1], w[3]);
+      } else if (bit == 8) {
+        lane_swap<8>(w[0], w[2]); lane_swap<8>(w[1], w[3]);
+      }
+      if (!r4 && sa < sb) { const double2 t = w[1]; w[1] = w[2]; w[2] = t; }
+    }
+    return;
+  }
 #pragma unroll
   for (int g = 0; g < NS; ++g)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = g * WC + lds_slot<MP>(sa < sb ? sa : sb, pt, stage_pos<MP>(sa, l, r));
+      const int i = g * WC + lds_slot<MP>(s, pt, stage_pos<MP>(sa, l, r));
       SFX_CHECK("lds exchange write", i, NS * WC);
       lds[i] = v[g][r];
     }
@@ -180,48 +251,58 @@ SFX_DEV void exchange(double2 (*v)[4], int sa, int sb, int pt, int l, double2* l
   for (int g = 0; g < NS; ++g)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = g * WC + lds_slot<MP>(sa < sb ? sa : sb, pt, stage_pos<MP>(sb, l, r));
+      const int i = g * WC + lds_slot<MP>(s, pt, stage_pos<MP>(sb, l, r));
       SFX_CHECK("lds exchange read", i, NS * WC);
       v[g][r] = lds[i];
     }
   SFX_WAVE_SYNC();
 }
 
-// Full inverse length-MP transform of NS signals (register arrays v[NS][4]),
-// exchanging in groups of at most G signals.
-template <int MP, int NS, int G>
-SFX_DEV void inverse_fft(double2 (&v)[NS][4], int pt, int l, double2* lds,
-                                            const double2* __restrict__ wMP) {
+// All stages of G signals.
+template <int MP, int G>
+SFX_DEV void inverse_fft_group(double2 (*v)[4], int pt, int l, double2* lds, const double2* __restrict__ wMP) {
   constexpr int NST = Shape<MP>::NST;
 #pragma unroll
   for (int s = 0; s < NST; ++s) {
 #pragma unroll
-    for (int g = 0; g < NS; ++g) inv_stage<MP>(s, l, v[g], wMP);
-    if (s + 1 < NST) {
-#pragma unroll
-      for (int g0 = 0; g0 < NS; g0 += G) {
-        if (g0 + G <= NS) exchange<MP, G>(&v[g0], s, s + 1, pt, l, lds);
-        else exchange<MP, (NS % G == 0 ? G : NS % G)>(&v[g0], s, s + 1, pt, l, lds);
-      }
-    }
+    for (int g = 0; g < G; ++g) inv_stage<MP>(s, l, v[g], wMP);
+    if (s + 1 < NST) exchange<MP, G>(v, s, s + 1, pt, l, lds);
   }
 }
-
-template <int MP, int NS, int G>
-SFX_DEV void forward_fft(double2 (&v)[NS][4], int pt, int l, double2* lds,
-                                            const double2* __restrict__ wMP) {
+template <int MP, int G>
+SFX_DEV void forward_fft_group(double2 (*v)[4], int pt, int l, double2* lds, const double2* __restrict__ wMP) {
   constexpr int NST = Shape<MP>::NST;
 #pragma unroll
   for (int s = NST - 1; s >= 0; --s) {
 #pragma unroll
-    for (int g = 0; g < NS; ++g) fwd_stage<MP>(s, l, v[g], wMP);
-    if (s > 0) {
+    for (int g = 0; g < G; ++g) fwd_stage<MP>(s, l, v[g], wMP);
+    if (s > 0) exchange<MP, G>(v, s, s - 1, pt, l, lds);
+  }
+}
+
+// Full inverse length-MP transform of NS signals (register arrays v[NS][4]), G
+// at a time: interleaving all of them hides no more latency and costs the
+// registers of their temporaries (scratch per lane of u.grad c at MP = 64 284
+// -> 60 bytes, of the point-tile cross-curl 68 -> 0; forward term at 200,704
+// triangles, M = 64, 4.78 -> 4.23 ms, u.grad c right-hand side at M = 24 0.97
+// -> 0.81 ms; the adjoint, which did not spill, 9.30 -> 9.37 ms).
+template <int MP, int NS, int G>
+SFX_DEV void inverse_fft(double2 (&v)[NS][4], int pt, int l, double2* lds, const double2* __restrict__ wMP) {
 #pragma unroll
-      for (int g0 = 0; g0 < NS; g0 += G) {
-        if (g0 + G <= NS) exchange<MP, G>(&v[g0], s, s - 1, pt, l, lds);
-        else exchange<MP, (NS % G == 0 ? G : NS % G)>(&v[g0], s, s - 1, pt, l, lds);
-      }
-    }
+  for (int g0 = 0; g0 < NS; g0 += G) {
+    if (g0 + G <= NS) inverse_fft_group<MP, G>(&v[g0], pt, l, lds, wMP);
+    else inverse_fft_group<MP, (NS % G == 0 ? G : NS % G)>(&v[g0], pt, l, lds, wMP);
+    SFX_SCHED_BARRIER();
+  }
+}
+
+template <int MP, int NS, int G>
+SFX_DEV void forward_fft(double2 (&v)[NS][4], int pt, int l, double2* lds, const double2* __restrict__ wMP) {
+#pragma unroll
+  for (int g0 = 0; g0 < NS; g0 += G) {
+    if (g0 + G <= NS) forward_fft_group<MP, G>(&v[g0], pt, l, lds, wMP);
+    else forward_fft_group<MP, (NS % G == 0 ? G : NS % G)>(&v[g0], pt, l, lds, wMP);
+    SFX_SCHED_BARRIER();
   }
 }
 

@@ -80,7 +80,7 @@ SFX_DEV void load_signal(const FftProdArgs& a, int64_t p, bool valid, int pt, in
   }
   // mode MP - m of slot r is held by lane (L - l) % L in slot 3 - r (l >= 1)
   // or 4 - r (l = 0, r >= 1); layout xf[(4 slot + j) * 64 + lane]
-  const int lane = pt * L + l, plane = pt * L + (L - l) % L;
+  const int lane = lane_at<MP>(pt, l), plane = lane_partner<MP>(pt, l);
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -215,12 +215,12 @@ constexpr size_t fftprod_smem_cplx(int wpb) { return 4 * MP + (size_t)wpb * 3 * 
 template <int MP, int OP>
 SFX_DEV void fftprod_body(const FftProdArgs& a, int tid, int64_t bid, int wpb, double2* smem) {
   using S = Shape<MP>;
-  constexpr int L = S::L, PW = S::PW;
+  constexpr int PW = S::PW;
   constexpr int NF = OpT<OP>::NF, NS = NF / 2, NO = OpT<OP>::NO;
   constexpr int NOC = (NO + 1) / 2;
   constexpr int GX = 3;                           // signals per LDS exchange
   const int wave = tid >> 6, lane = tid & 63;
-  const int pt = lane / L, l = lane % L;
+  const int pt = lane_pt<MP>(lane), l = lane_l<MP>(lane);
   // twiddle tables staged in LDS once per work-group: wN (3 MP) then wMP (MP)
   double2* tw = smem;
   for (int i = tid; i < 4 * MP; i += 64 * wpb) tw[i] = (i < 3 * MP) ? a.wN[i] : a.wMP[i - 3 * MP];

@@ -284,9 +284,7 @@ SFX_DEV void nodal_store(const NodalFetch<NC, MP, NW>& f, int tid, double* nod, 
 // Layout xf[f * 64 + lane]: consecutive lanes, consecutive doubles.
 template <int NF, int MP>
 SFX_DEV void partner_swap(const double (&own)[NF], double (&par)[NF], int pt, int l, double* xf) {
-  constexpr int L = MP / 4;
-  const int me_ = pt * L + l;
-  const int pa = pt * L + ((L - l) % L);
+  const int me_ = lane_at<MP>(pt, l), pa = lane_partner<MP>(pt, l);
 #pragma unroll
   for (int f = 0; f < NF; ++f) { SFX_CHECK("field swap", f * 64 + me_, 64 * NF); xf[f * 64 + me_] = own[f]; }
   SFX_WAVE_SYNC();
@@ -439,7 +437,7 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
   constexpr int GX = 2;
   constexpr int NT = 64 * NW;
   const int wave = tid >> 6, lane = tid & 63;
-  const int pt = lane / L, l = lane % L;
+  const int pt = lane_pt<MP>(lane), l = lane_l<MP>(lane);
   double* smd = reinterpret_cast<double*>(smem);
 
   // ---- per work-group tables

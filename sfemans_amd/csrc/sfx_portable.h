@@ -27,6 +27,8 @@ struct sfx_d4 {
 sfx_d4 sfx_emu_mfma_f64(double a, double b, const sfx_d4& c);
 #define SFX_MFMA_F64(a, b, c) sfx_emu_mfma_f64((a), (b), (c))
 #define SFX_UNIFORM(x) (x)
+void sfx_emu_lane_swap(double& a, double& b, int bit);
+#define SFX_LANE_SWAP(a, b, bit) sfx_emu_lane_swap((a), (b), (bit))
 #define SFX_WAVE_SYNC() sfx_emu_wave_sync()
 #define SFX_OPAQUE(x) do { } while (0)
 #define SFX_OPAQUE_S(x) do { } while (0)
@@ -56,6 +58,36 @@ typedef double sfx_d4 __attribute__((ext_vector_type(4)));
 #define SFX_MFMA_F64(a, b, c) __builtin_amdgcn_mfma_f64_16x16x4f64((a), (b), (c), 0, 0, 0)
 // An int that is the same in every lane of the wave, as a scalar.
 #define SFX_UNIFORM(x) __builtin_amdgcn_readfirstlane(x)
+// Transpose the pair (a, b) with a lane bit (32, 16, 8 or 4): lanes whose bit is
+// 0 keep a and get the a of lane + BIT in b; lanes whose bit is 1 keep b and get
+// the b of lane - BIT in a.
+template <int BIT>
+__device__ __forceinline__ void sfx_lane_swap(double& a, double& b) {
+  union { double d; unsigned u[2]; } x, y;
+  x.d = a;
+  y.d = b;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if constexpr (BIT == 32) {
+      const auto r = __builtin_amdgcn_permlane32_swap(x.u[i], y.u[i], false, false);
+      x.u[i] = r[0];
+      y.u[i] = r[1];
+    } else if constexpr (BIT == 16) {
+      const auto r = __builtin_amdgcn_permlane16_swap(x.u[i], y.u[i], false, false);
+      x.u[i] = r[0];
+      y.u[i] = r[1];
+    } else {
+      // DPP row_shr / row_shl by BIT, written to the banks of 4 lanes whose bit is 1 / 0
+      constexpr int HI = BIT == 8 ? 0xc : 0xa, LO = BIT == 8 ? 0x3 : 0x5;
+      const unsigned p = x.u[i], q = y.u[i];
+      x.u[i] = __builtin_amdgcn_update_dpp(p, q, 0x110 + BIT, 0xf, HI, false);
+      y.u[i] = __builtin_amdgcn_update_dpp(q, p, 0x100 + BIT, 0xf, LO, false);
+    }
+  }
+  a = x.d;
+  b = y.d;
+}
+#define SFX_LANE_SWAP(a, b, bit) sfx_lane_swap<bit>((a), (b))
 // Hide a value's origin from the optimizer, so that what is computed from it
 // is recomputed where it is used instead of being kept live (or spilled)
 // across a long stretch of code.  Emits no instruction.

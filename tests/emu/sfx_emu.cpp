@@ -38,6 +38,17 @@ sfx_d4 sfx_emu_mfma_f64(double a, double b, const sfx_d4& c) {
   g_wave_bar->arrive_and_wait();
   return d;
 }
+// transposition of (a, b) with a lane bit: every lane of the wave calls it together
+void sfx_emu_lane_swap(double& a, double& b, int bit) {
+  g_wave_ab[0][g_lane] = a;
+  g_wave_ab[1][g_lane] = b;
+  g_wave_bar->arrive_and_wait();
+  const bool one = (g_lane & bit) != 0;
+  const double x = one ? g_wave_ab[1][g_lane - bit] : a, y = one ? b : g_wave_ab[0][g_lane + bit];
+  g_wave_bar->arrive_and_wait();
+  a = x;
+  b = y;
+}
 void sfx_emu_oob(const char* what, long long idx, long long n, const char* file, int line) {
   std::fprintf(stderr, "SFX_EMU out of bounds: %s index %lld not in [0,%lld) at %s:%d\n", what, idx, n, file, line);
   std::fflush(stderr);
