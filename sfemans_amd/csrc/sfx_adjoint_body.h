@@ -86,7 +86,7 @@ struct AdjLds {
   static constexpr int PK2 = PARK ? (LDS_DOUBLES - 2 * LY::BIG - BIGD) / NT : 0;
   static constexpr int PK = PK1 + PK2;
   static constexpr int TOTAL = LY::BIG + (BIGD + PK2 * NT + 1) / 2;   // double2 units
-  static_assert(!PARK || (PK2 >= 0 && 2 * TOTAL <= LDS_DOUBLES), "parking exceeds the LDS");
+  static_assert(PK2 >= 0 && 2 * TOTAL <= LDS_DOUBLES, "LDS of the work-group");
 };
 
 // Parked slot f (0 <= f < PK) of lane t.

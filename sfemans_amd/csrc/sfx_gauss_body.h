@@ -96,7 +96,10 @@ struct GaussLds {
   static constexpr int GEO = MODE + MP;                 // per element 6 nodes (r,z)
   static constexpr int NID = GEO + E * 6;               // per element 6 node indices (int)
   static constexpr int BIG = NID + (E * 6 + 3) / 4;
-  static constexpr int ROW6 = L * 6 + 2;                // doubles per node slot, 6 columns
+  // doubles per node slot, 6 columns: 16-byte reads of the modes of one element
+  // (48 bytes apart) and of the next one (6 rows on) then miss each other's banks;
+  // shorter rows at small MP, whose many elements fill the LDS
+  static constexpr int ROW6 = L * 6 + (L >= 8 ? 6 : 2);
   static constexpr int ROW2 = L * 2 + 2;                // doubles per node slot, 2 columns
   static constexpr int NOD6 = E * 6 * ROW6;             // doubles of one staged 6-column field
   static constexpr int NOD2 = E * 6 * ROW2;
@@ -128,6 +131,7 @@ struct GaussCfg {
   // chunk buffers when not staging all at once: two where they fit
   static constexpr int NBUF = GaussLds<MP, NW, 2, NCB>::TOTAL * 16 <= GAUSS_LDS_BYTES ? 2 : 1;
   using LY = GaussLds<MP, NW, ALL ? 4 : NBUF, NCB>;
+  static_assert(LY::TOTAL * 16 <= GAUSS_LDS_BYTES, "LDS of the work-group");
 };
 
 struct GaussGeom {
@@ -137,33 +141,49 @@ struct GaussGeom {
   double iray;
 };
 
-// Interpolation at one Gauss point and one mode from a staged node row set:
-// values and reference derivatives, then the affine map to (r, z) derivatives
-// (dw = J^{-T} dd, gauss_points_2d.F90:108-121).
-// nod: staged block; s0: first node slot of the element; row: doubles per slot.
-template <int NC, int MP>
-SFX_DEV void interp_mode(const double* nod, int s0, int row, int mi, const GaussGeom& g,
-                         double (&W)[NC], double (&Dr)[NC], double (&Dz)[NC]) {
-  double Dx[NC], Dy[NC];
+// Values of NC columns at one Gauss point and one mode from a staged node row
+// set: s0 first node slot of the element, row doubles per slot, mode-major
+// (nod[slot*row + mode*NC + column], read two columns at a time).
+template <int NC>
+SFX_DEV void interp_value(const double* nod, int s0, int row, int mi, const GaussGeom& g, double (&W)[NC]) {
 #pragma unroll
-  for (int k = 0; k < NC; ++k) { W[k] = 0; Dx[k] = 0; Dy[k] = 0; }
+  for (int k = 0; k < NC; ++k) W[k] = 0;
 #pragma unroll
   for (int n = 0; n < 6; ++n) {
-    // column-major slot: the lanes of a point read consecutive modes
-    const double* v = nod + (s0 + n) * row + mi;
-    const double wn = g.w[n], dx = g.d[2 * n], dy = g.d[2 * n + 1];
+    const double2* v = reinterpret_cast<const double2*>(nod + (s0 + n) * row + mi * NC);
+    const double wn = g.w[n];
 #pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      const double x = v[k * (MP / 4)];
-      W[k] = fma(wn, x, W[k]);
-      Dx[k] = fma(dx, x, Dx[k]);
-      Dy[k] = fma(dy, x, Dy[k]);
+    for (int k = 0; k < NC / 2; ++k) {
+      const double2 x = v[k];
+      W[2 * k] = fma(wn, x.x, W[2 * k]);
+      W[2 * k + 1] = fma(wn, x.y, W[2 * k + 1]);
     }
   }
+}
+
+// Values, and the derivatives d/dr of the columns in RMASK and d/dz of those in
+// ZMASK.  The shape derivatives are mapped to (r, z) node by node (dw = J^{-T}
+// dd, gauss_points_2d.F90:108-121): 24 operations and one FMA per node for each
+// derivative that is used, where mapping the reference derivatives of every
+// column takes two per node and 24 operations (132 -> 108 for the curl).
+template <int NC, int RMASK, int ZMASK>
+SFX_DEV void interp_mode(const double* nod, int s0, int row, int mi, const GaussGeom& g,
+                         double (&W)[NC], double (&Dr)[NC], double (&Dz)[NC]) {
 #pragma unroll
-  for (int k = 0; k < NC; ++k) {
-    Dr[k] = fma(g.a11, Dx[k], g.a12 * Dy[k]);
-    Dz[k] = fma(g.a21, Dx[k], g.a22 * Dy[k]);
+  for (int k = 0; k < NC; ++k) W[k] = Dr[k] = Dz[k] = 0;
+#pragma unroll
+  for (int n = 0; n < 6; ++n) {
+    const double2* v = reinterpret_cast<const double2*>(nod + (s0 + n) * row + mi * NC);
+    const double wn = g.w[n], dx = g.d[2 * n], dy = g.d[2 * n + 1];
+    const double dr = fma(g.a11, dx, g.a12 * dy), dz = fma(g.a21, dx, g.a22 * dy);
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      const double2 x2 = v[k / 2];
+      const double x = (k & 1) ? x2.y : x2.x;
+      W[k] = fma(wn, x, W[k]);
+      if ((RMASK >> k) & 1) Dr[k] = fma(dr, x, Dr[k]);
+      if ((ZMASK >> k) & 1) Dz[k] = fma(dz, x, Dz[k]);
+    }
   }
 }
 
@@ -225,57 +245,67 @@ SFX_DEV T pick(const T (&v)[N], int i) {
   return r;
 }
 
-// Stage the nodal values of modes [c*L, c*L+L) of a (np, NC, M) array for
-// the E elements of this work-group: nod[(slot)*row + mi*NC + k].
+// Staging of the nodal values of modes [c*L, c*L+L) of a (np, NC, M) array for
+// the E elements of this work-group, mode-major: nod[slot*row + mode*NC + k].
+// These are Q = NC L consecutive planes of the array; a thread keeps one node
+// slot and takes every R-th plane (several slots, every plane, where the
+// work-group has fewer threads than slots), so that its addresses advance by a
+// constant and its LDS stores have constant offsets.  The forward kernel is
+// bound by vector instruction issue (67 % of its cycles), and numbering slots,
+// columns and modes through one index took about 24 of them per value.
+// Measured with the interpolation below (16-byte LDS reads, only the
+// derivatives that are used) and the stores of staged outputs at constant
+// strides, at 200,704 triangles, M = 64: 4453 -> 3820 vector instructions per
+// wave, forward term 4.22 -> 3.81 ms; tangent at 99,856 triangles, M = 32, 3.57
+// -> 3.25 ms.
 template <int NC, int MP, int NW>
 struct NodalFetch {
-  static constexpr int TOT = GaussLds<MP>::E * 6 * NC * (MP / 4);
-  static constexpr int NT = 64 * NW;
-  static constexpr int IT = (TOT + NT - 1) / NT;
-  double v[IT];
+  static constexpr int S = GaussLds<MP>::E * 6, NT = 64 * NW, Q = NC * (MP / 4);
+  static constexpr int SI = (S + NT - 1) / NT;          // slots per thread
+  static constexpr int R = SI > 1 ? 1 : NT / S;         // threads per slot
+  static constexpr int IT = (Q + R - 1) / R;
+  double v[SI][IT];
 };
 
-// Issue the loads of chunk c (modes [c*L, c*L+L)) of a (np, NC, M) nodal array
-// for the E elements of this work-group into registers; unconditional loads at
-// clamped indices, so they all issue back to back and overlap other work.
+// Issue the loads of chunk c into registers: unconditional (planes past the
+// last mode read the slot's first value, which no interpolation uses), so that
+// they all issue back to back and overlap other work.
 template <int NC, int MP, int NW>
 SFX_DEV void nodal_fetch(const GaussArgs& a, const double* X, int64_t nX, int64_t e0, int c, int tid,
                          const int* nid, NodalFetch<NC, MP, NW>& f) {
-  using NF_ = NodalFetch<NC, MP, NW>;
-  constexpr int L = MP / 4, S = GaussLds<MP>::E * 6;
+  using F = NodalFetch<NC, MP, NW>;
 #pragma unroll
-  for (int it = 0; it < NF_::IT; ++it) {
-    const int idx = tid + it * NF_::NT;
-    const int id = idx < NF_::TOT ? idx : 0;
-    const int s = id % S;
-    const int rest = id / S;
-    const int k = rest % NC;
-    const int mi = rest / NC;
-    const int64_t e = e0 + s / 6;
-    const int m = c * L + mi;
-    const bool ok = idx < NF_::TOT && e < a.me && m < a.M;
-    const int64_t gi = (int64_t)nid[s] + a.np * (k + (int64_t)NC * (m < a.M ? m : 0));
-    SFX_CHECK("nodal load", gi, nX);
-    const double x = X[gi];
-    f.v[it] = ok ? x : 0.0;
+  for (int si = 0; si < F::SI; ++si) {
+    const int t = tid + si * F::NT;
+    const bool on = F::SI > 1 ? t < F::S : t < F::S * F::R;
+    const int s = on ? t % F::S : 0, q0 = on && F::SI == 1 ? t / F::S : 0;
+    const double* base = X + nid[s];
+    const double* p = base + a.np * (int64_t)(c * F::Q + q0);
+    const int left = NC * a.M - c * F::Q - q0;          // planes of this thread before the last mode's end
+#pragma unroll
+    for (int it = 0; it < F::IT; ++it, p += a.np * F::R) {
+      const double* b = it * F::R < left ? p : base;
+      SFX_CHECK("nodal load", b - X, nX);
+      f.v[si][it] = *b;
+    }
   }
 }
 
-// Store a fetched chunk to LDS: nod[slot*row + k*L + mi] (columns of L
-// modes, so that the lanes of a point read consecutive doubles).
+// Store a fetched chunk to LDS.
 template <int NC, int MP, int NW>
 SFX_DEV void nodal_store(const NodalFetch<NC, MP, NW>& f, int tid, double* nod, int row) {
-  using NF_ = NodalFetch<NC, MP, NW>;
-  constexpr int S = GaussLds<MP>::E * 6;
+  using F = NodalFetch<NC, MP, NW>;
 #pragma unroll
-  for (int it = 0; it < NF_::IT; ++it) {
-    const int idx = tid + it * NF_::NT;
-    if (idx < NF_::TOT) {
-      const int s = idx % S;
-      const int rest = idx / S;
-      const int li = s * row + (rest % NC) * (MP / 4) + rest / NC;
-      SFX_CHECK("nodal stage", li, S * row);
-      nod[li] = f.v[it];
+  for (int si = 0; si < F::SI; ++si) {
+    const int t = tid + si * F::NT;
+    const int s = t % F::S, q0 = F::SI == 1 ? t / F::S : 0;
+    if (F::SI > 1 ? t >= F::S : (F::S * F::R < F::NT && t >= F::S * F::R)) continue;
+    double* d = nod + s * row + q0;
+#pragma unroll
+    for (int it = 0; it < F::IT; ++it) {
+      if ((it + 1) * F::R > F::Q && q0 + it * F::R >= F::Q) continue;   // the last, partial round
+      SFX_CHECK("nodal stage", s * row + q0 + it * F::R, F::S * row);
+      d[it * F::R] = f.v[si][it];
     }
   }
 }
@@ -322,25 +352,22 @@ SFX_DEV void pass_fields(const GaussArgs& a, const double* nodA, const double* n
   const double mr = mval * g.iray;
   if constexpr (V == GV_CROSS_CURL || V == GV_PAIRS || V == GV_CURL_CROSS) {
     double W[6], Dr[6], Dz[6], R[6];
-    interp_mode<6, MP>(nodA, s0, LY::ROW6, mi, g, W, Dr, Dz);
+    interp_mode<6, 0x3c, 0x0f>(nodA, s0, LY::ROW6, mi, g, W, Dr, Dz);   // the derivatives curl6 uses
     curl6(W, Dr, Dz, mr, g.iray, R);
     if constexpr (V == GV_CROSS_CURL) {
       // precession: RotV += 2 Omega (mode 1: r_c and theta_s, mode 0: z_c)
       if (mval == 1.0) { R[0] += a.om[0]; R[3] += a.om[1]; }
       if (mval == 0.0) { R[4] += a.om[2]; }
     }
-    if ((V == GV_PAIRS || V == GV_CURL_CROSS) && nodB != nullptr) {
-      double Drb[6], Dzb[6];
-      interp_mode<6, MP>(nodB, s0, LY::ROW6, mi, g, W, Drb, Dzb);
-    }
+    if ((V == GV_PAIRS || V == GV_CURL_CROSS) && nodB != nullptr) interp_value<6>(nodB, s0, LY::ROW6, mi, g, W);
     // signals (R_r, R_theta), (R_z, W_r), (W_theta, W_z)
     F[0] = R[0]; F[1] = R[1]; F[2] = R[2]; F[3] = R[3];
     F[4] = R[4]; F[5] = R[5]; F[6] = W[0]; F[7] = W[1];
     F[8] = W[2]; F[9] = W[3]; F[10] = W[4]; F[11] = W[5];
   } else {  // GV_UGRADC
     double W[6], Dr[6], Dz[6], C[2], Cr[2], Cz[2];
-    interp_mode<6, MP>(nodA, s0, LY::ROW6, mi, g, W, Dr, Dz);
-    interp_mode<2, MP>(nodB, s0, LY::ROW2, mi, g, C, Cr, Cz);
+    interp_mode<6, 0x03, 0x30>(nodA, s0, LY::ROW6, mi, g, W, Dr, Dz);   // the divergence
+    interp_mode<2, 0x03, 0x03>(nodB, s0, LY::ROW2, mi, g, C, Cr, Cz);
     const double d0 = Dr[0] + W[0] * g.iray + mr * W[3] + Dz[4];
     const double d1 = Dr[1] + W[1] * g.iray - mr * W[2] + Dz[5];
     // signals (G_r, G_theta), (G_z, W_r), (W_theta, W_z), (Div, C)
@@ -702,18 +729,22 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
     }
   }
   if constexpr (SOUT) {
+    // a thread keeps one point and takes every L-th plane
     constexpr int TP = PT ? NW * PW : 7 * E, SR = TP + 1;
-    const double* st = big;
+    static_assert(NT == TP * L, "planes per round");
+    const int lp = tid % TP, P0 = tid / TP;
+    const int64_t pg = p0 + lp;
+    const double* st = big + P0 * SR + lp;
+    double* o = a.Vout + pg + a.G * (int64_t)P0;
     SFX_SYNC();
-    const int items = 2 * NO * a.M * TP;
-    for (int it = tid; it < items; it += NT) {
-      const int lp = it % TP, P = it / TP;
-      const int64_t pg = p0 + lp;
-      if (pg >= 7 * a.me) continue;
-      SFX_CHECK("out stage read", P * SR + lp, 2 * NO * MP * SR);
-      SFX_CHECK("gauss out", pg + a.G * (int64_t)P, a.nout);
-      if (V == GV_CURL_CROSS && a.accum) a.Vout[pg + a.G * (int64_t)P] += st[P * SR + lp];
-      else a.Vout[pg + a.G * (int64_t)P] = st[P * SR + lp];
+    if (pg < 7 * a.me) {
+#pragma unroll 4
+      for (int P = P0; P < 2 * NO * a.M; P += L, st += L * SR, o += a.G * L) {
+        SFX_CHECK("out stage read", st - big, 2 * NO * MP * SR);
+        SFX_CHECK("gauss out", o - a.Vout, a.nout);
+        if (V == GV_CURL_CROSS && a.accum) *o += *st;
+        else *o = *st;
+      }
     }
   }
   if constexpr (RHS) {
