@@ -168,7 +168,7 @@ def wl_mhd(torch, args):
         # written and read back are re-traffic
         Phase("rhs_ns_3x3", lambda: NL.rhs_ns_3x3(mesh, modes, work, v1m, fsrc, pr, pinc, v145, v236, welem),
               G * 6 * M * 8 + npn * 16 * M * 8 + npn * 6 * M * 8 + m.me * 7 * 8 + 12 * 6 * m.me + npn * 16,
-              G * M * (6 * 2 * 6 + 16 * 6 * 2), "rhs_ns_elem_kernel + rhs_gather_kernel",
+              G * M * (6 * 2 * 6 + 16 * 6 * 2), "rhs_ns_tile_kernel<false> + rhs_gather_kernel",
               overhead=2 * 36 * m.me * M * 8),
         Phase("u_x_B_nodes", lambda: FP.FFT_PAR_CROSS_PROD_DCL(None, u, B, uxb), 3 * npn * 6 * M * 8,
               npn * fft_flops_per_point(M, 6, 3, 9), "fftprod_kernel<64,CROSS>"),
@@ -204,7 +204,7 @@ def wl_nsrhs(torch, args):
         Phase("rhs_ns_3x3_tensor",
               lambda: NL.rhs_ns_3x3(mesh, modes, rotv, v1m, fsrc, pr, pinc, v145, v236, welem, opt_tensor=tens),
               rest + G * 18 * M * 8, G * M * (6 * 2 * 6 + 16 * 6 * 2 + 6 * 6 * 6 + 20),
-              "rhs_ns_elem_kernel<true> + rhs_gather_kernel", overhead=2 * 36 * m.me * M * 8),
+              "rhs_ns_tile_kernel<true> + rhs_gather_kernel", overhead=2 * 36 * m.me * M * 8),
     ]
     cfg = {"workload": "full per-mode NS right-hand side with rhs_3x3's tensor (LES / variable viscosity), "
                        "224x448 P2 mesh (200,704 triangles, 1,404,928 Gauss points), m_max=64: "

@@ -12,13 +12,14 @@ __global__ void __launch_bounds__(256) rhs_elem_kernel(RhsArgs a) {
 }
 
 template <bool TENSOR>
-__global__ void __launch_bounds__(256) rhs_ns_elem_kernel(RhsArgs a) {
-  rhs_ns_elem_body<TENSOR>(a, xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x);
+__global__ void __launch_bounds__(RNS_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) rhs_ns_tile_kernel(RhsArgs a) {
+  __shared__ __attribute__((aligned(16))) double smem[rns_smem_doubles<TENSOR>()];
+  rhs_ns_tile_body<TENSOR>(a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x), smem);
 }
 
 // The Gauss values of the NS right-hand side before the penalty product.
 __global__ void __launch_bounds__(256) rhs_ns_gauss_kernel(RhsArgs a) {
-  rhs_ns_elem_body<false, true>(a, xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x);
+  rhs_ns_gauss_body(a, xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x);
 }
 
 __global__ void __launch_bounds__(GATHER_THREADS) rhs_gather_kernel(RhsArgs a) {
@@ -64,12 +65,11 @@ hipError_t launch_qs00_gather(const RhsArgs& a, hipStream_t st) {
 
 // Full NS right-hand side fused with its element share, then the gather.
 hipError_t launch_rhs_ns(const RhsArgs& a, hipStream_t st) {
-  const int64_t ne = a.me > 0 && a.M > 0 ? elem_items(a.me, a.M) : 0, nn = a.np * a.M;
-  if (ne > 0) {
-    if (a.tens)
-      hipLaunchKernelGGL(rhs_ns_elem_kernel<true>, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL(rhs_ns_elem_kernel<false>, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, st, a);
+  const int64_t nn = a.np * a.M, nt = a.me > 0 && a.M > 0 ? rns_blocks(a.me, a.M) : 0;
+  if (nt > 0x7fffffffLL) return hipErrorInvalidValue;
+  if (nt > 0) {
+    if (a.tens) hipLaunchKernelGGL(rhs_ns_tile_kernel<true>, dim3((unsigned)nt), dim3(RNS_THREADS), 0, st, a);
+    else hipLaunchKernelGGL(rhs_ns_tile_kernel<false>, dim3((unsigned)nt), dim3(RNS_THREADS), 0, st, a);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nn == 0) return e;

@@ -40,7 +40,7 @@ struct RhsArgs {
   double* vect;             // (np, M)
   double* elo;              // per-element nodal contributions, index ((6e+i)*6 + k)*M + m
   int64_t n_rhs, n_ff, n_ffg, n_out, n_adj, n_elo;
-  // full NS right-hand side (rhs_ns_elem_body); a null field counts as zero
+  // full NS right-hand side (rhs_ns_tile_body); a null field counts as zero
   const double* rr;         // (2, np) node coordinates
   const int32_t* lmode;     // (M) mode numbers
   const double* v1m;        // (np, 6, M) time-derivative term
@@ -118,7 +118,7 @@ SFX_DEV void rhs_elem_body(const RhsArgs& a, int64_t gid) {
 
 // Full explicit NS right-hand side of rhs_ns_gauss_3x3 without the penalty
 // options (SOURCES/SOLVER/computing_rhs_gauss.F90:7-146) fused with the
-// element share of rhs_3x3, one thread per (element, mode) (elem_item):
+// element share of rhs_3x3:
 //   rhs(l, :) = (ft + fp_inc + fs - rotv_v(7e+l, :)) + fp         (:100, :145)
 // (rsign = -1; with rsign = +1 and the other fields absent it is rhs_3x3's
 // own rhs_in, so the kernel also serves rhs_3x3 with opt_tensor)
@@ -132,12 +132,228 @@ SFX_DEV void rhs_elem_body(const RhsArgs& a, int64_t gid) {
 // with f_tensor the 1/r and mode terms (row k/2 of T, its cos columns for
 // even k, sin for odd).
 // The Gauss array rhs_gauss is never stored.
-// With GOUT the kernel writes the Gauss values (ft + fp_inc + fs - rotv_v,
-// minus the imposed velocity on its slot) to gout instead of assembling them:
-// the first step of the penalty branch, whose product with the penalty
-// function mixes the modes at each Gauss point (computing_rhs_gauss.F90:124-129).
-template <bool TENSOR, bool GOUT = false>
-SFX_DEV void rhs_ns_elem_body(const RhsArgs& a, int64_t gid) {
+//
+// What bounds it: HBM (rotv_v and the tensor are 192 bytes per Gauss point and
+// mode).  A work-group takes RNS_E elements and RNS_MC modes of them, one mode
+// at a time: one thread per Gauss point loads rotv_v and the tensor (224
+// consecutive points of each plane, whole lines), one per (element, node) the
+// nodal fields, which are added at the nodes (V1m + ff, P + P_inc) and
+// interpolated from LDS; each point's weights of the shape values and of the
+// reference derivatives (18 numbers, as in the adjoint) go to LDS, and one
+// thread per (element, component) sums them for the six nodes, keeping RNS_MC
+// modes so that it stores 64-byte runs.  (One thread per (element, mode) with all
+// of its fields in registers took 418 registers, one wave per SIMD, and each of
+// its loads touched 40 lines: 1.4 TB/s, 6.15 ms with the gather at 102,720
+// triangles, M = 48, against 3.04 ms, 3.8 TB/s in this kernel.)
+constexpr int RNS_E = 32, RNS_MC = 8, RNS_THREADS = 256;
+constexpr int RNS_PT = 7 * RNS_E;              // Gauss points
+constexpr int RNS_EROW = 6 * 8 + 2;            // doubles per element of the staged nodal sums (8 per node)
+constexpr int RNS_SK = RNS_PT + 2;             // doubles per weight
+template <bool TENSOR>
+constexpr int rns_smem_doubles() { return 2 * RNS_E * RNS_EROW + (TENSOR ? 18 : 6) * RNS_SK + 128; }
+inline int64_t rns_blocks(int64_t me, int M) {
+  return ((me + RNS_E - 1) / RNS_E) * (int64_t)((M + RNS_MC - 1) / RNS_MC);
+}
+
+template <bool TENSOR>
+SFX_DEV void rhs_ns_tile_body(const RhsArgs& a, int tid, int64_t bid, double* smem) {
+  const int nmc = (a.M + RNS_MC - 1) / RNS_MC;
+  const int64_t e0 = (bid / nmc) * RNS_E;      // the mode chunks of one set of elements are neighbours
+  const int m0 = (int)(bid % nmc) * RNS_MC, m1 = m0 + RNS_MC < a.M ? m0 + RNS_MC : a.M;
+  double* nod = smem;                          // two buffers: a slow thread still reads the other mode's
+  double* red = nod + 2 * RNS_E * RNS_EROW;
+  double* tab = red + (TENSOR ? 18 : 6) * RNS_SK;
+  for (int i = tid; i < 126; i += RNS_THREADS) tab[i] = a.tab[i];
+
+  // this thread's node slot, Gauss point and (element, component)
+  const bool nslot = tid < 6 * RNS_E && e0 + tid / 6 < a.me;
+  const int64_t node = nslot ? (int64_t)a.jj[6 * e0 + tid] - 1 : 0;
+  const int el = tid / 7, lg = tid % 7;
+  const bool point = tid < RNS_PT && e0 + el < a.me;
+  const int64_t p = point ? 7 * e0 + tid : 0;
+  const int ke = tid % RNS_E, kc = tid / RNS_E;
+  const bool sums = tid < 6 * RNS_E && e0 + ke < a.me;
+  double a11 = 0, a12 = 0, a21 = 0, a22 = 0, iray = 0, wl = 0;
+  SFX_SYNC();
+  const double* w = tab + 6 * (point ? lg : 0);
+  const double* d = tab + 42 + 12 * (point ? lg : 0);
+  if (point) {
+    double rn[6], zn[6], ray = 0;
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {
+      const int64_t jn = (int64_t)a.jj[6 * (e0 + el) + n] - 1;
+      SFX_CHECK("rr load", 2 * jn + 1, 2 * a.np);
+      rn[n] = a.rr[2 * jn];
+      zn[n] = a.rr[2 * jn + 1];
+      ray = fma(rn[n], w[n], ray);
+    }
+    p2_inverse_jacobian(rn, zn, d, a11, a12, a21, a22);
+    iray = 1.0 / ray;
+    wl = a.wgt[p];
+  }
+  double acc[RNS_MC][6];
+#pragma unroll
+  for (int q = 0; q < RNS_MC; ++q)
+#pragma unroll
+    for (int i = 0; i < 6; ++i) acc[q][i] = 0.0;
+
+#pragma unroll
+  for (int q = 0; q < RNS_MC; ++q) {
+    const int m = m0 + q;
+    if (m >= m1) continue;                     // uniform over the work-group
+    // ---- loads of this mode
+    double rv[6], T[TENSOR ? 3 : 1][6];
+    if (point) {
+      const int64_t g0 = p + a.G * 6 * (int64_t)m;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        SFX_CHECK("rotv load", g0 + a.G * k, a.rhs ? a.n_rhs : 1 << 30);
+        rv[k] = a.rhs ? a.rhs[g0 + a.G * k] : 0.0;
+        if constexpr (TENSOR) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            SFX_CHECK("tensor load", c + 3 * (g0 + a.G * k), a.n_tens);
+            T[c][k] = a.tens[c + 3 * (g0 + a.G * k)];
+          }
+        }
+      }
+    }
+    double* nb = nod + (q & 1) * RNS_E * RNS_EROW;
+    if (nslot) {
+      double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      const int64_t i6 = node + a.np * 6 * (int64_t)m, i2 = node + a.np * 2 * (int64_t)m;
+      if (a.v1m) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          SFX_CHECK("V1m load", i6 + a.np * k, a.n_v1m);
+          s[k] = a.v1m[i6 + a.np * k];
+        }
+      }
+      if (a.fsrc) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          SFX_CHECK("ff load", i6 + a.np * k, a.n_fsrc);
+          s[k] += a.fsrc[i6 + a.np * k];
+        }
+      }
+      if (a.pres) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          SFX_CHECK("P load", i2 + a.np * k, a.n_pres);
+          s[6 + k] = a.pres[i2 + a.np * k];
+        }
+      }
+      if (a.pinc) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          SFX_CHECK("P_inc load", i2 + a.np * k, a.n_pinc);
+          s[6 + k] += a.pinc[i2 + a.np * k];
+        }
+      }
+      if (a.imp && m == a.imp_slot) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          SFX_CHECK("imposed velocity load", node + a.np * k, a.n_imp);
+          s[k] += a.isign * a.imp[node + a.np * k];
+        }
+      }
+      double2* o = reinterpret_cast<double2*>(nb + (tid / 6) * RNS_EROW + (tid % 6) * 8);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = make_double2(s[2 * k], s[2 * k + 1]);
+    }
+    SFX_SYNC();
+    // ---- the right-hand side at this point: weights of the shape values and
+    // of d/dx, d/dy
+    if (point) {
+      const double mv = (double)a.lmode[m];
+      double f[6], pv[2] = {0, 0}, pr[2] = {0, 0}, pz[2] = {0, 0};
+#pragma unroll
+      for (int k = 0; k < 6; ++k) f[k] = 0.0;
+#pragma unroll
+      for (int n = 0; n < 6; ++n) {
+        const double2* s = reinterpret_cast<const double2*>(nb + el * RNS_EROW + n * 8);
+        const double wn = w[n], dx = d[2 * n], dy = d[2 * n + 1];
+        const double dr = fma(a11, dx, a12 * dy), dz = fma(a21, dx, a22 * dy);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const double2 x = s[k];
+          f[2 * k] = fma(wn, x.x, f[2 * k]);
+          f[2 * k + 1] = fma(wn, x.y, f[2 * k + 1]);
+        }
+        const double2 x = s[3];
+        pv[0] = fma(wn, x.x, pv[0]); pv[1] = fma(wn, x.y, pv[1]);
+        pr[0] = fma(dr, x.x, pr[0]); pr[1] = fma(dr, x.y, pr[1]);
+        pz[0] = fma(dz, x.x, pz[0]); pz[1] = fma(dz, x.y, pz[1]);
+      }
+      const double mr = mv * iray;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) f[k] = f[k] + a.rsign * rv[k];
+      f[0] -= pr[0]; f[1] -= pr[1];
+      f[2] -= mr * pv[1]; f[3] += mr * pv[0];
+      f[4] -= pz[0]; f[5] -= pz[1];
+      double* o = red + tid;
+      if constexpr (TENSOR) {
+        f[0] += (-mv * T[0][3] + T[1][2]) * iray;
+        f[1] += (mv * T[0][2] + T[1][3]) * iray;
+        f[2] += (-T[0][2] - mv * T[1][3]) * iray;
+        f[3] += (-T[0][3] + mv * T[1][2]) * iray;
+        f[4] -= T[2][3] * mr;
+        f[5] += T[2][2] * mr;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          const double tr = T[k / 2][k % 2] * wl, tz = T[k / 2][4 + k % 2] * wl;
+          o[(3 * k) * RNS_SK] = f[k] * wl;
+          o[(3 * k + 1) * RNS_SK] = fma(a11, tr, a21 * tz);
+          o[(3 * k + 2) * RNS_SK] = fma(a12, tr, a22 * tz);
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) o[k * RNS_SK] = f[k] * wl;
+      }
+    }
+    SFX_SYNC();
+    // ---- sums over the element's points, the tables through scalar registers
+    if (sums) {
+      constexpr int KW = TENSOR ? 3 : 1;
+      const SFX_KARG double* tb = (const SFX_KARG double*)a.tab;
+      SFX_OPAQUE_S(tb);
+      const double* src = red + KW * kc * RNS_SK + 7 * ke;
+#pragma unroll
+      for (int l = 0; l < 7; ++l) {
+        double v[KW];
+#pragma unroll
+        for (int j = 0; j < KW; ++j) v[j] = src[j * RNS_SK + l];
+#pragma unroll
+        for (int n = 0; n < 6; ++n) {
+          if constexpr (TENSOR) {
+            const double dx = tb[42 + 2 * (n + 6 * l)], dy = tb[42 + 2 * (n + 6 * l) + 1];
+            acc[q][n] = fma(tb[n + 6 * l], v[0], fma(dx, v[1], fma(dy, v[2], acc[q][n])));
+          } else {
+            acc[q][n] = fma(tb[n + 6 * l], v[0], acc[q][n]);
+          }
+        }
+      }
+    }
+  }
+  if (sums) {
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {
+      const int64_t o = ((6 * (e0 + ke) + n) * 6 + kc) * (int64_t)a.M + m0;
+#pragma unroll
+      for (int q = 0; q < RNS_MC; ++q) {
+        if (m0 + q >= m1) continue;
+        SFX_CHECK("elo store", o + q, a.n_elo);
+        a.elo[o + q] = acc[q][n];
+      }
+    }
+  }
+}
+
+// The Gauss values ft + fp_inc + fs - rotv_v, minus the imposed velocity on its
+// slot, to gout, one thread per (element, mode) (elem_item): the first step of
+// the penalty branch, whose product with the penalty function mixes the modes
+// at each Gauss point (computing_rhs_gauss.F90:124-129).
+SFX_DEV void rhs_ns_gauss_body(const RhsArgs& a, int64_t gid) {
   int64_t e;
   int m;
   elem_item(gid, a.M, e, m);
@@ -152,7 +368,7 @@ SFX_DEV void rhs_ns_elem_body(const RhsArgs& a, int64_t gid) {
     zn[n] = a.rr[2 * j[n] + 1];
   }
   const double mv = (double)a.lmode[m];
-  double V[6][6], F[6][6], P[6][2], Q[6][2];
+  double V[6][6], F[6][6], Q[6][2];
 #pragma unroll
   for (int n = 0; n < 6; ++n) {
 #pragma unroll
@@ -166,18 +382,11 @@ SFX_DEV void rhs_ns_elem_body(const RhsArgs& a, int64_t gid) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int64_t i2 = j[n] + a.np * (k + 2 * (int64_t)m);
-      SFX_CHECK("P load", i2, a.pres ? a.n_pres : 1 << 30);
       SFX_CHECK("P_inc load", i2, a.pinc ? a.n_pinc : 1 << 30);
-      P[n][k] = a.pres ? a.pres[i2] : 0.0;
       Q[n][k] = a.pinc ? a.pinc[i2] : 0.0;
     }
   }
   const bool imposed = a.imp && m == a.imp_slot;
-  double loc[6][6];
-#pragma unroll
-  for (int i = 0; i < 6; ++i)
-#pragma unroll
-    for (int k = 0; k < 6; ++k) loc[i][k] = 0.0;
 #pragma unroll
   for (int l = 0; l < 7; ++l) {
     const double* w = a.tab + 6 * l;
@@ -187,7 +396,7 @@ SFX_DEV void rhs_ns_elem_body(const RhsArgs& a, int64_t gid) {
     double a11, a12, a21, a22;
     p2_inverse_jacobian(rn, zn, d, a11, a12, a21, a22);
     double ray = 0, ft[6] = {0, 0, 0, 0, 0, 0}, fs[6] = {0, 0, 0, 0, 0, 0};
-    double pv[2] = {0, 0}, px[2] = {0, 0}, py[2] = {0, 0}, qv[2] = {0, 0}, qx[2] = {0, 0}, qy[2] = {0, 0};
+    double qv[2] = {0, 0}, qx[2] = {0, 0}, qy[2] = {0, 0};
 #pragma unroll
     for (int n = 0; n < 6; ++n) {
       ray = fma(rn[n], w[n], ray);
@@ -198,27 +407,19 @@ SFX_DEV void rhs_ns_elem_body(const RhsArgs& a, int64_t gid) {
       }
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        pv[k] = fma(P[n][k], w[n], pv[k]);
-        px[k] = fma(P[n][k], d[2 * n], px[k]);
-        py[k] = fma(P[n][k], d[2 * n + 1], py[k]);
         qv[k] = fma(Q[n][k], w[n], qv[k]);
         qx[k] = fma(Q[n][k], d[2 * n], qx[k]);
         qy[k] = fma(Q[n][k], d[2 * n + 1], qy[k]);
       }
     }
-    double fp[6], fq[6];
+    double fq[6];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      fp[k] = -fma(a11, px[k], a12 * py[k]);
-      fp[4 + k] = -fma(a21, px[k], a22 * py[k]);
       fq[k] = -fma(a11, qx[k], a12 * qy[k]);
       fq[4 + k] = -fma(a21, qx[k], a22 * qy[k]);
     }
-    fp[2] = -pv[1] / ray * mv;
-    fp[3] = pv[0] / ray * mv;
     fq[2] = -qv[1] / ray * mv;
     fq[3] = qv[0] / ray * mv;
-    const double wl = a.wgt[7 * e + l];
     const int64_t gi = 7 * e + l + a.G * 6 * (int64_t)m;
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
@@ -235,79 +436,10 @@ SFX_DEV void rhs_ns_elem_body(const RhsArgs& a, int64_t gid) {
         }
         base = base + a.isign * iv;
       }
-      if constexpr (GOUT) {
-        SFX_CHECK("gauss store", gi + a.G * k, a.n_gout);
-        a.gout[gi + a.G * k] = base;
-      } else {
-        const double r = (base + fp[k]) * wl;
-#pragma unroll
-        for (int i = 0; i < 6; ++i) loc[i][k] = fma(w[i], r, loc[i][k]);
-      }
+      SFX_CHECK("gauss store", gi + a.G * k, a.n_gout);
+      a.gout[gi + a.G * k] = base;
     }
   }
-  if constexpr (GOUT) return;
-  // The tensor terms in a second pass over the Gauss points, once the nodal
-  // fields are dead: the two passes never hold both in registers.
-  if constexpr (TENSOR) {
-    // the node coordinates again (from L2), so that they are not held over
-    // the first pass: the opaque pointer keeps these loads from being merged
-    // with the first ones
-    const double* rr2 = a.rr;
-    const int32_t* jj2 = a.jj;
-    SFX_OPAQUE_S(rr2);
-    SFX_OPAQUE_S(jj2);
-#pragma unroll
-    for (int n = 0; n < 6; ++n) {
-      const int64_t jn = (int64_t)jj2[6 * e + n] - 1;
-      rn[n] = rr2[2 * jn];
-      zn[n] = rr2[2 * jn + 1];
-    }
-#pragma unroll 1
-    for (int l = 0; l < 7; ++l) {
-      const double* w = a.tab + 6 * l;
-      const double* d = a.tab + 42 + 12 * l;
-      double a11, a12, a21, a22;
-      p2_inverse_jacobian(rn, zn, d, a11, a12, a21, a22);
-      double ray = 0;
-#pragma unroll
-      for (int n = 0; n < 6; ++n) ray = fma(rn[n], w[n], ray);
-      const double wl = a.wgt[7 * e + l];
-      const int64_t gi = 7 * e + l + a.G * 6 * (int64_t)m;
-      double T[3][6];
-#pragma unroll
-      for (int t = 0; t < 6; ++t)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const int64_t it = k + 3 * (gi + a.G * t);
-          SFX_CHECK("tensor load", it, a.n_tens);
-          T[k][t] = a.tens[it];
-        }
-      double fT[6];
-      fT[0] = (-mv * T[0][3] + T[1][2]) / ray;
-      fT[1] = (mv * T[0][2] + T[1][3]) / ray;
-      fT[2] = (-T[0][2] - mv * T[1][3]) / ray;
-      fT[3] = (-T[0][3] + mv * T[1][2]) / ray;
-      fT[4] = -T[2][3] * mv / ray;
-      fT[5] = T[2][2] * mv / ray;
-#pragma unroll
-      for (int i = 0; i < 6; ++i) {
-        const double dr = fma(a11, d[2 * i], a12 * d[2 * i + 1]) * wl;
-        const double dz = fma(a21, d[2 * i], a22 * d[2 * i + 1]) * wl;
-        const double wi = w[i] * wl;
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-          loc[i][k] = fma(wi, fT[k], fma(dr, T[k / 2][k % 2], fma(dz, T[k / 2][4 + k % 2], loc[i][k])));
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 6; ++i)
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      const int64_t o = ((6 * e + i) * 6 + k) * a.M + m;
-      SFX_CHECK("elo store", o, a.n_elo);
-      a.elo[o] = loc[i][k];
-    }
 }
 
 // vb_145 / vb_236 of work-group bid: the nodes' element contributions summed

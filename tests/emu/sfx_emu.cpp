@@ -290,7 +290,7 @@ extern "C" int emu_rhs_ns_gauss(const int32_t* jj, const double* rr, int64_t me,
   a.imp = imp; a.imp_slot = imp ? imp_slot : -1; a.isign = -1.0; a.gout = gout;
   a.n_rhs = a.G * 6 * (int64_t)M; a.n_v1m = a.n_fsrc = np * 6 * (int64_t)M; a.n_pinc = np * 2 * (int64_t)M;
   a.n_imp = np * 6; a.n_gout = a.G * 6 * (int64_t)M;
-  for (int64_t g = 0; g < elem_items(me, M); ++g) rhs_ns_elem_body<false, true>(a, g);
+  for (int64_t g = 0; g < elem_items(me, M); ++g) rhs_ns_gauss_body(a, g);
   return 0;
 }
 
@@ -315,12 +315,12 @@ extern "C" int emu_rhs_ns(const int32_t* jj, const double* rr, int64_t me, int64
   a.n_rhs = a.G * 6 * (int64_t)M; a.n_v1m = a.n_fsrc = np * 6 * (int64_t)M; a.n_pres = a.n_pinc = np * 2 * (int64_t)M;
   a.n_tens = 3 * a.n_rhs;
   a.n_out = np * 3 * (int64_t)M; a.n_elo = 36 * me * (int64_t)M;
-  for (int64_t g = 0; g < elem_items(me, M); ++g) {
-    if (tens)
-      rhs_ns_elem_body<true>(a, g);
-    else
-      rhs_ns_elem_body<false>(a, g);
-  }
+  if (tens)
+    run_grid(rns_blocks(me, M), RNS_THREADS, (rns_smem_doubles<true>() + 1) / 2,
+             [&](int t, int64_t b, double2* sm) { rhs_ns_tile_body<true>(a, t, b, reinterpret_cast<double*>(sm)); });
+  else
+    run_grid(rns_blocks(me, M), RNS_THREADS, (rns_smem_doubles<false>() + 1) / 2,
+             [&](int t, int64_t b, double2* sm) { rhs_ns_tile_body<false>(a, t, b, reinterpret_cast<double*>(sm)); });
   run_grid((np + GATHER_NODES - 1) / GATHER_NODES, GATHER_THREADS, (gather_tile_doubles<6>() + 1) / 2,
            [&](int t, int64_t b, double2* sm) { rhs_gather_block(a, b, t, reinterpret_cast<double*>(sm)); });
   return 0;
