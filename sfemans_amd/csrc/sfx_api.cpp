@@ -197,7 +197,7 @@ int run_fftprod_host(int op, const char* name, const double* V1, const double* V
   if (rc) return rc;
   if ((e = hipDeviceSynchronize()) != hipSuccess) return hip_fail(e, name);
   double t2 = now_s();
-  if ((e = hipMemcpy(Vout, d3, no * 8, hipMemcpyDeviceToHost)) != hipSuccess) return hip_fail(e, "D2H");
+  if ((e = copy_out(Vout, d3, no * 8)) != hipSuccess) return hip_fail(e, "D2H");
   double t3 = now_s();
   if (temps) { temps[0] = (t1 - t0) + (t3 - t2); temps[1] = t2 - t1; }
   return SFX_OK;
@@ -215,7 +215,11 @@ const char* sfx_version(void) { return "sfx 0.1 (gfx950, FP64)"; }
 
 int sfx_stream_release(void* stream) {
   clear_err();
-  return release_stream_scratch((hipStream_t)stream);
+  const int rc = release_stream_scratch((hipStream_t)stream);
+  if (rc || stream) return rc;
+  // the host-pointer entry points run on the null stream
+  const hipError_t e = release_hostcopy();
+  return e == hipSuccess ? SFX_OK : hip_fail(e, "sfx_stream_release");
 }
 
 int sfx_init(int32_t device) {

@@ -36,6 +36,8 @@ int get_twiddles(int MP, Twiddles* tw);
 int staging(int slot, size_t bytes, void** out);
 int stream_scratch(int slot, size_t bytes, hipStream_t st, void** out);
 int release_stream_scratch(hipStream_t st);
+hipError_t copy_out(void* h, const void* d, size_t n);
+hipError_t release_hostcopy();
 double now_s();
 int check_modes(const char* name, int64_t np, int32_t m_max_c, int32_t m_max_pad);
 int check_procs(const char* name, int64_t np, int32_t nb_procs, int64_t bloc_size);

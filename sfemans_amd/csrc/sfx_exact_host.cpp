@@ -354,7 +354,7 @@ static int to_dev(int slot, const double* h, size_t n, void** d) {
 static int from_dev(double* h, const void* d, size_t n) {
   hipError_t e = hipDeviceSynchronize();
   if (e != hipSuccess) return hip_fail(e, "exact-grid product");
-  e = n ? hipMemcpy(h, d, n * 8, hipMemcpyDeviceToHost) : hipSuccess;
+  e = n ? copy_out(h, d, n * 8) : hipSuccess;
   return e == hipSuccess ? SFX_OK : hip_fail(e, "D2H");
 }
 

@@ -264,7 +264,7 @@ static int run_gauss_host(int variant, const char* nm, sfx_mesh_t mesh, const in
                      nin > 1 ? (const double*)din[1] : nullptr, nin > 1 ? in[1].nc : 0, npass ? &ps : nullptr,
                      (const double*)dH, (double*)dO, ncout, om, nullptr);
   if (rc) return rc;
-  if ((e = hipMemcpy(out, dO, nO * 8, hipMemcpyDeviceToHost)) != hipSuccess) return hip_fail(e, "D2H");
+  if ((e = copy_out(out, dO, nO * 8)) != hipSuccess) return hip_fail(e, "D2H");
   return SFX_OK;
 }
 
@@ -525,7 +525,7 @@ int sfx_nl_adjoint(sfx_mesh_t mesh, const int32_t* list_mode, int32_t m_max_c, c
   if ((rc = sfx_nl_adjoint_dev(mesh, (const int32_t*)dL, m_max_c, (const double*)dU, (const double*)dY, (double*)dE,
                                (double*)dO, nullptr)))
     return rc;
-  if ((e = hipMemcpy(dbar, dO, nU * 8, hipMemcpyDeviceToHost)) != hipSuccess) return hip_fail(e, "D2H");
+  if ((e = copy_out(dbar, dO, nU * 8)) != hipSuccess) return hip_fail(e, "D2H");
   return SFX_OK;
 }
 
@@ -691,8 +691,8 @@ int sfx_rhs_3x3_mode(sfx_mesh_t mesh, int32_t mode, const double* rhs_in, const 
   }
   if (nB && (rc = sfx_rhs_3x3_bdy_dev(mesh, 1, (const double*)db, (double*)d1, (double*)d2, 1.0, nullptr)))
     return rc;
-  if ((e = hipMemcpy(vb_145, d1, nN * 8, hipMemcpyDeviceToHost)) != hipSuccess) return hip_fail(e, "D2H");
-  if ((e = hipMemcpy(vb_236, d2, nN * 8, hipMemcpyDeviceToHost)) != hipSuccess) return hip_fail(e, "D2H");
+  if ((e = copy_out(vb_145, d1, nN * 8)) != hipSuccess) return hip_fail(e, "D2H");
+  if ((e = copy_out(vb_236, d2, nN * 8)) != hipSuccess) return hip_fail(e, "D2H");
   return SFX_OK;
 }
 
@@ -709,8 +709,8 @@ int sfx_rhs_3x3(sfx_mesh_t mesh, int32_t mode, const double* rhs_in, double* vb_
   hipError_t e;
   if ((e = hipMemcpy(dr, rhs_in, nG * 8, hipMemcpyHostToDevice)) != hipSuccess) return hip_fail(e, "H2D");
   if ((rc = rhs3x3_dev(mesh, 1, (const double*)dr, (double*)d1, (double*)d2, 1.0, (double*)dw, nullptr))) return rc;
-  if ((e = hipMemcpy(vb_145, d1, nN * 8, hipMemcpyDeviceToHost)) != hipSuccess) return hip_fail(e, "D2H");
-  if ((e = hipMemcpy(vb_236, d2, nN * 8, hipMemcpyDeviceToHost)) != hipSuccess) return hip_fail(e, "D2H");
+  if ((e = copy_out(vb_145, d1, nN * 8)) != hipSuccess) return hip_fail(e, "D2H");
+  if ((e = copy_out(vb_236, d2, nN * 8)) != hipSuccess) return hip_fail(e, "D2H");
   return SFX_OK;
 }
 
@@ -747,7 +747,7 @@ int sfx_qs_00_gauss(sfx_mesh_t mesh, const double* heat_capa, const double* ff, 
   if ((rc = sfx_qs_00_gauss_dev(mesh, 1, (const double*)dh, (const double*)df, (const double*)dg, (double*)dw,
                                 (double*)dv, nullptr)))
     return rc;
-  if ((e = hipMemcpy(vect, dv, nN * 8, hipMemcpyDeviceToHost)) != hipSuccess) return hip_fail(e, "D2H");
+  if ((e = copy_out(vect, dv, nN * 8)) != hipSuccess) return hip_fail(e, "D2H");
   return SFX_OK;
 }
 
