@@ -247,9 +247,16 @@ SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem)
   double* tab = smd + 2 * LY::TAB;
   double* lmode = smd + 2 * LY::MODE;
   double2* geo = smem + LY::GEO;
-  int* nid = reinterpret_cast<int*>(smem + LY::NID);
   const int64_t e0 = bid * E;
-  gauss_prologue<MP, NW>(a, tid, e0, smem);
+  // the first chunk of the base fields leaves with the tables' loads
+  NodalSlots<MP, NW> slots;
+  NodalFetch<6, MP, NW> fa, fb;
+  auto fetch = [&](int c) {
+    nodal_fetch<6, MP, NW>(a, a.U, a.nU, c, tid, slots, fa);
+    if (SPLIT) nodal_fetch<6, MP, NW>(a, A.UB, A.nUB, c, tid, slots, fb);
+  };
+  nodal_slots<MP, NW>(a, e0, tid, slots);
+  gauss_prologue<MP, NW>(a, tid, e0, smem, [&] { fetch(0); });
   SFX_SYNC();
   const double2* wN = tw;
   const double2* wMP = tw + 3 * MP;
@@ -282,9 +289,6 @@ SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem)
 #pragma unroll
       for (int r = 0; r < 4; ++r) { Z[gi][s][r] = make_double2(0, 0); B[gi][s][r] = make_double2(0, 0); }
   {
-    NodalFetch<6, MP, NW> fa, fb;
-    nodal_fetch<6, MP, NW>(a, a.U, a.nU, e0, 0, tid, nid, fa);
-    if (SPLIT) nodal_fetch<6, MP, NW>(a, A.UB, A.nUB, e0, 0, tid, nid, fb);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       // chunk c into buffer c % 2 (chunk c - 2 there was interpolated by
@@ -292,10 +296,7 @@ SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem)
       double* nodA = big + (c & 1) * (SPLIT ? 2 : 1) * LY::NOD6;
       nodal_store<6, MP, NW>(fa, tid, nodA, LY::ROW6);
       if (SPLIT) nodal_store<6, MP, NW>(fb, tid, nodA + LY::NOD6, LY::ROW6);
-      if (c < 3) {
-        nodal_fetch<6, MP, NW>(a, a.U, a.nU, e0, c + 1, tid, nid, fa);
-        if (SPLIT) nodal_fetch<6, MP, NW>(a, A.UB, A.nUB, e0, c + 1, tid, nid, fb);
-      }
+      if (c < 3) fetch(c + 1);
       SFX_SYNC();
       const int m = c * L + l;
 #pragma unroll

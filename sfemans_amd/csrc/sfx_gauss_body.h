@@ -258,28 +258,50 @@ SFX_DEV T pick(const T (&v)[N], int i) {
 // strides, at 200,704 triangles, M = 64: 4453 -> 3820 vector instructions per
 // wave, forward term 4.22 -> 3.81 ms; tangent at 99,856 triangles, M = 32, 3.57
 // -> 3.25 ms.
-template <int NC, int MP, int NW>
-struct NodalFetch {
-  static constexpr int S = GaussLds<MP>::E * 6, NT = 64 * NW, Q = NC * (MP / 4);
+template <int MP, int NW>
+struct NodalSlots {
+  static constexpr int S = GaussLds<MP>::E * 6, NT = 64 * NW;
   static constexpr int SI = (S + NT - 1) / NT;          // slots per thread
   static constexpr int R = SI > 1 ? 1 : NT / S;         // threads per slot
+  int node[SI];                                         // node (from 0) of the thread's slots
+};
+template <int NC, int MP, int NW>
+struct NodalFetch {
+  using SL = NodalSlots<MP, NW>;
+  static constexpr int S = SL::S, NT = SL::NT, SI = SL::SI, R = SL::R;
+  static constexpr int Q = NC * (MP / 4);
   static constexpr int IT = (Q + R - 1) / R;
   double v[SI][IT];
 };
+
+// The thread's slots of the E elements from e0 on (node 0 past the last element).
+template <int MP, int NW>
+SFX_DEV void nodal_slots(const GaussArgs& a, int64_t e0, int tid, NodalSlots<MP, NW>& f) {
+  using F = NodalSlots<MP, NW>;
+#pragma unroll
+  for (int si = 0; si < F::SI; ++si) {
+    const int t = tid + si * F::NT;
+    const bool on = F::SI > 1 ? t < F::S : t < F::S * F::R;
+    const int s = on ? t % F::S : 0;
+    const int64_t e = e0 + s / 6;
+    const int n = a.jj[e < a.me ? 6 * e + s % 6 : 0];
+    f.node[si] = e < a.me ? n - 1 : 0;
+  }
+}
 
 // Issue the loads of chunk c into registers: unconditional (planes past the
 // last mode read the slot's first value, which no interpolation uses), so that
 // they all issue back to back and overlap other work.
 template <int NC, int MP, int NW>
-SFX_DEV void nodal_fetch(const GaussArgs& a, const double* X, int64_t nX, int64_t e0, int c, int tid,
-                         const int* nid, NodalFetch<NC, MP, NW>& f) {
+SFX_DEV void nodal_fetch(const GaussArgs& a, const double* X, int64_t nX, int c, int tid,
+                         const NodalSlots<MP, NW>& sl, NodalFetch<NC, MP, NW>& f) {
   using F = NodalFetch<NC, MP, NW>;
 #pragma unroll
   for (int si = 0; si < F::SI; ++si) {
     const int t = tid + si * F::NT;
     const bool on = F::SI > 1 ? t < F::S : t < F::S * F::R;
-    const int s = on ? t % F::S : 0, q0 = on && F::SI == 1 ? t / F::S : 0;
-    const double* base = X + nid[s];
+    const int q0 = on && F::SI == 1 ? t / F::S : 0;
+    const double* base = X + sl.node[si];
     const double* p = base + a.np * (int64_t)(c * F::Q + q0);
     const int left = NC * a.M - c * F::Q - q0;          // planes of this thread before the last mode's end
 #pragma unroll
@@ -380,9 +402,10 @@ SFX_DEV void pass_fields(const GaussArgs& a, const double* nodA, const double* n
 
 // Per work-group tables in LDS: twiddles, reference-element tables, mode
 // numbers, node coordinates and node numbers of the E elements.  All loads
-// issue together (clamped indices), then the LDS stores.
-template <int MP, int NW>
-SFX_DEV void gauss_prologue(const GaussArgs& a, int tid, int64_t e0, double2* smem) {
+// issue together (clamped indices), then what `issue` loads for the caller,
+// then the LDS stores.
+template <int MP, int NW, class Issue>
+SFX_DEV void gauss_prologue(const GaussArgs& a, int tid, int64_t e0, double2* smem, const Issue& issue) {
   using LY = GaussLds<MP, NW>;
   constexpr int E = LY::E, NT = 64 * NW;
   double* smd = reinterpret_cast<double*>(smem);
@@ -414,6 +437,7 @@ SFX_DEV void gauss_prologue(const GaussArgs& a, int tid, int64_t e0, double2* sm
       SFX_CHECK("rr load", 2 * (int64_t)node[it] + 1, 2 * a.np);
       rz[it] = make_double2(a.rr[2 * (int64_t)node[it]], a.rr[2 * (int64_t)node[it] + 1]);
     }
+    issue();
 #pragma unroll
     for (int it = 0; it < ITW; ++it) {
       const int i = tid + it * NT;
@@ -475,16 +499,10 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
   int* nid = reinterpret_cast<int*>(smem + LY::NID);
   const int64_t p0 = PT ? bid * (int64_t)(NW * PW) : bid * (int64_t)(7 * E);   // first Gauss point
   const int64_t e0 = p0 / 7;
-  gauss_prologue<MP, NW>(a, tid, e0, smem);
-  static_assert(126 <= NT && MP <= NT, "prologue assumes one table entry per thread");
-  SFX_SYNC();
-  const double2* wN = tw;
-  const double2* wMP = tw + 3 * MP;
 
   // ---- this lane's Gauss point in each of the wave's groups (group wave + NW*gi)
-  GaussGeom g[NG];
   bool has[NG], valid[NG];
-  int el[NG];
+  int el[NG], lq[NG];
   int64_t p[NG];
   double hc[NG];
 #pragma unroll
@@ -494,12 +512,51 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
     const int lp = (has[gi] ? grp : 0) * PW + pt;    // local point
     const int64_t pg = p0 + lp;
     el[gi] = (int)(pg / 7 - e0);
-    const int lg = (int)(pg % 7);
     p[gi] = pg;
     valid[gi] = has[gi] && pg < 7 * a.me;
-    gauss_geom(geo + 6 * el[gi], tab, valid[gi] ? lg : 0, g[gi]);
-    hc[gi] = (V == GV_UGRADC && valid[gi]) ? a.heat_capa[e0 + el[gi]] : 1.0;
+    lq[gi] = valid[gi] ? (int)(pg % 7) : 0;
   }
+
+  // The first chunks' loads depend on the connectivity alone: they leave with
+  // those of the tables, ahead of the first barrier and the geometry, and a
+  // chunk is two ahead of its use where a second work-group shares the CU or
+  // two fields are staged (forward term at 200,704 triangles, M = 64, 3.81 ->
+  // 3.61 ms, of whose 59,000 cycles a wave spent 19,000 waiting for chunks;
+  // tangent at 99,856 triangles, M = 32, 3.28 -> 3.23 ms, with one ahead 3.24).
+  // The element sums keep one ahead: two take 6.79 ms against 6.54 at 90,300
+  // triangles, M = 100, and 0.754 against 0.745 for u.grad c, M = 24.
+  constexpr bool EARLY = !ALL && V != GV_PAIRS;
+  constexpr int NCB = (V == GV_UGRADC) ? 2 : 6;
+  constexpr int DEP = ALL ? 4 : (PT || V == GV_CURL_CROSS) ? 2 : 1;   // chunks in registers
+  NodalSlots<MP, NW> slots;
+  NodalFetch<6, MP, NW> fa[DEP];
+  NodalFetch<NCB, MP, NW> fb[DEP];
+  auto fetch = [&](const double* XA, int64_t nXA, const double* XB, int64_t nXB, bool useB, int c) {
+    nodal_fetch<6, MP, NW>(a, XA, nXA, c, tid, slots, fa[c % DEP]);
+    if (useB) nodal_fetch<NCB, MP, NW>(a, XB, nXB, c, tid, slots, fb[c % DEP]);
+  };
+  const double* XA = V == GV_CURL_CROSS ? a.pc[0] : a.U;
+  const double* XB = V == GV_CURL_CROSS ? a.pv[0] : a.U2;
+  int64_t nXA = V == GV_CURL_CROSS ? a.npc[0] : a.nU, nXB = V == GV_CURL_CROSS ? a.npv[0] : a.nU2;
+  double coef = V == GV_CURL_CROSS ? a.coef[0] : 1.0;
+  bool useB = V == GV_UGRADC || (V == GV_CURL_CROSS && XB != XA);
+  nodal_slots<MP, NW>(a, e0, tid, slots);
+  gauss_prologue<MP, NW>(a, tid, e0, smem, [&] {
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi)
+      hc[gi] = V == GV_UGRADC ? a.heat_capa[valid[gi] ? e0 + el[gi] : 0] : 1.0;
+    if (EARLY)
+#pragma unroll
+      for (int c = 0; c < DEP; ++c) fetch(XA, nXA, XB, nXB, useB, c);
+  });
+  static_assert(126 <= NT && MP <= NT, "prologue assumes one table entry per thread");
+  SFX_SYNC();
+  const double2* wN = tw;
+  const double2* wMP = tw + 3 * MP;
+
+  GaussGeom g[NG];
+#pragma unroll
+  for (int gi = 0; gi < NG; ++gi) gauss_geom(geo + 6 * el[gi], tab, lq[gi], g[gi]);
 
   double* big = smd + 2 * LY::BIG;
   double* xf = big + LY::XCH + (size_t)wave * LY::RW;
@@ -533,16 +590,8 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
 #pragma unroll
           for (int r = 0; r < 4; ++r) { Z[gs][s][r] = make_double2(0, 0); B[gs][s][r] = make_double2(0, 0); }
       // nodal arrays of this pass: A (6 columns) and B (6 or 2 columns, or none)
-      constexpr int NCB = (V == GV_UGRADC) ? 2 : 6;
       // (the pass entries are picked with selects: indexing the argument
       // arrays with the loop counter would copy them to scratch memory)
-      const double* XA = a.U;
-      const double* XB = a.U2;
-      int64_t nXA = a.nU, nXB = a.nU2;
-      double coef = 1.0;
-      if (V == GV_CURL_CROSS) {
-        XA = a.pc[0]; XB = a.pv[0]; nXA = a.npc[0]; nXB = a.npv[0]; coef = a.coef[0];
-      }
       if (V == GV_PAIRS) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -553,26 +602,20 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
           nXB = on ? a.npv[k] : nXB;
           coef = on ? a.coef[k] : coef;
         }
+        useB = XB != XA;
       }
-      const bool useB = (V == GV_UGRADC) || ((V == GV_PAIRS || V == GV_CURL_CROSS) && XB != XA);
-      NodalFetch<6, MP, NW> fa[ALL ? 4 : 1];
-      NodalFetch<NCB, MP, NW> fb[ALL ? 4 : 1];
+      if constexpr (!EARLY) {
+#pragma unroll
+        for (int c = 0; c < DEP; ++c) fetch(XA, nXA, XB, nXB, useB, c);
+      }
       if constexpr (ALL) {
         // every chunk at once: all loads issue back to back, one barrier
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          nodal_fetch<6, MP, NW>(a, XA, nXA, e0, c, tid, nid, fa[c]);
-          if (useB) nodal_fetch<NCB, MP, NW>(a, XB, nXB, e0, c, tid, nid, fb[c]);
-        }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           nodal_store<6, MP, NW>(fa[c], tid, big + c * LY::NODC, LY::ROW6);
           if (useB) nodal_store<NCB, MP, NW>(fb[c], tid, big + c * LY::NODC + LY::NOD6, NCB == 6 ? LY::ROW6 : LY::ROW2);
         }
         SFX_SYNC();
-      } else {
-        nodal_fetch<6, MP, NW>(a, XA, nXA, e0, 0, tid, nid, fa[0]);
-        if (useB) nodal_fetch<NCB, MP, NW>(a, XB, nXB, e0, 0, tid, nid, fb[0]);
       }
       constexpr int NBUF = GaussCfg<MP, V, NW, STAGE_ALL>::NBUF;
 #pragma unroll
@@ -582,16 +625,13 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
         if constexpr (!ALL) {
           // two buffers: chunk c into buffer c % 2 (its previous chunk, c - 2,
           // was interpolated by every wave before the last barrier), start
-          // fetching chunk c + 1, and one barrier makes chunk c visible.  One
+          // fetching chunk c + DEP, and one barrier makes chunk c visible.  One
           // buffer: wait until every wave is done with chunk c - 1 first.
           if (NBUF == 1) SFX_SYNC();
-          nodal_store<6, MP, NW>(fa[0], tid, nodA, LY::ROW6);
-          if (useB) nodal_store<NCB, MP, NW>(fb[0], tid, nodB, NCB == 6 ? LY::ROW6 : LY::ROW2);
+          nodal_store<6, MP, NW>(fa[c % DEP], tid, nodA, LY::ROW6);
+          if (useB) nodal_store<NCB, MP, NW>(fb[c % DEP], tid, nodB, NCB == 6 ? LY::ROW6 : LY::ROW2);
           if (NBUF == 1) SFX_SYNC();
-          if (c < 3) {
-            nodal_fetch<6, MP, NW>(a, XA, nXA, e0, c + 1, tid, nid, fa[0]);
-            if (useB) nodal_fetch<NCB, MP, NW>(a, XB, nXB, e0, c + 1, tid, nid, fb[0]);
-          }
+          if (c + DEP < 4) fetch(XA, nXA, XB, nXB, useB, c + DEP);
           if (NBUF == 2) SFX_SYNC();
         }
         const int m = c * L + l;
@@ -624,7 +664,10 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
         if (!pick(has, gi)) continue;
         double2 y[3 * NSIG][4];
 #pragma unroll
-        for (int s = 0; s < NSIG; ++s) prestep<MP>(Z[gs][s], B[gs][s], l, y[3 * s], y[3 * s + 1], y[3 * s + 2], wN);
+        for (int s = 0; s < NSIG; ++s) {
+          prestep<MP>(Z[gs][s], B[gs][s], l, y[3 * s], y[3 * s + 1], y[3 * s + 2], wN);
+          if (V == GV_UGRADC && MP > 4) SFX_SCHED_BARRIER();   // with 4 signals, so that no register spills
+        }
         inverse_fft<MP, 3 * NSIG, GX>(y, pt, l, lds, wMP);
 #pragma unroll
         for (int j1 = 0; j1 < 3; ++j1)
