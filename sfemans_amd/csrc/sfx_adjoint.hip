@@ -3,8 +3,12 @@
 
 namespace sfx {
 
-template <int MP, bool SPLIT, int NW = adjoint_waves<MP, SPLIT>()>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NW), waves_per_simd(NW))))
+template <int MP, bool SPLIT>
+constexpr int adjoint_occupancy() { return adjoint_half<MP, SPLIT>() ? 2 : 1; }
+
+template <int MP, bool SPLIT, int NW = ADJOINT_WAVES>
+__global__ void __launch_bounds__(64 * NW)
+__attribute__((amdgpu_waves_per_eu(adjoint_occupancy<MP, SPLIT>(), adjoint_occupancy<MP, SPLIT>())))
 adjoint_kernel(AdjArgs a) {
   extern __shared__ double2 smem[];
   adjoint_body<MP, SPLIT, NW>(a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x), smem);
@@ -17,8 +21,8 @@ __global__ void __launch_bounds__(GATHER_THREADS) adjoint_gather_kernel(GatherAr
 
 template <int MP, bool SPLIT>
 static hipError_t launch_mp(const AdjArgs& a, hipStream_t st) {
-  constexpr int NW = adjoint_waves<MP, SPLIT>();
-  constexpr int E = GaussLds<MP, NW>::E;
+  constexpr int NW = ADJOINT_WAVES;
+  constexpr int E = adjoint_elems<MP, SPLIT>();
   const int64_t nblk = (a.g.me + E - 1) / E;
   if (nblk == 0) return hipSuccess;
   const size_t shmem = (size_t)AdjLds<MP, SPLIT, NW>::TOTAL * sizeof(double2);

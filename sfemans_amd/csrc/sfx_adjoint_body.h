@@ -38,28 +38,35 @@ struct AdjArgs {
 // weights of the two outputs apart.
 template <bool SPLIT> struct AdjRed { static constexpr int K = SPLIT ? 24 : 18; };
 
-// Waves per work-group of the adjoint kernel (see gauss_waves): 7 (256
-// registers, the parking form) for the convective form at 16 <= MP <= 128,
-// 4 (512 registers) elsewhere.  Measured at 200,704 triangles, 7 against 4
-// waves: M = 16 2.23 / 2.56 ms, M = 32 4.92 / 5.97, M = 128 25.9 / 29.6
-// (M = 64 was the first size moved to 7).
+// Half tiles of the adjoint kernel (see gauss_rhs_half): 4 waves with one group
+// each in 256 registers (the parking form), two work-groups per CU, where the
+// layout fits in half the LDS; elsewhere 4 waves with two groups each in 512
+// registers.  Half tiles against what stood there, convective form: 0.80 / 0.98
+// ms at MP = 4, 0.84 / 1.10 at 8 (both against 512 registers), 0.91 / 0.96 at 16,
+// 0.68 / 0.76 at 64, 0.86 / 0.94 at 128 (against 7 waves with one group each; a
+// wave waited 13,000 of 100,000 cycles at the barrier before the sums, three SIMDs
+// holding two waves and one holding one); split form, against 512 registers: 1.18
+// / 1.79 ms at MP = 8, 1.27 / 1.64 at 16, 1.31 / 1.68 at 32, 1.33 / 1.79 at 64.
 template <int MP, bool SPLIT>
-constexpr int adjoint_waves() { return (!SPLIT && MP >= 16 && MP <= 128) ? 7 : 4; }
+constexpr bool adjoint_half() { return SPLIT ? MP >= 8 && MP <= 64 : MP <= 128; }
+template <int MP, bool SPLIT>
+constexpr int adjoint_elems() { return adjoint_half<MP, SPLIT>() ? 128 / MP : gauss_elems<MP>(); }
+constexpr int ADJOINT_WAVES = 4;
 
 template <int MP, bool SPLIT, int NW>
 struct AdjLds {
-  using LY = GaussLds<MP, NW>;
+  using LY = GaussLds<MP, NW, 1, 6, adjoint_elems<MP, SPLIT>()>;
   static constexpr int NT = 64 * NW;
-  // Parking (convective form on 7 waves, 256 registers per lane): the base
-  // spectra wait in LDS while pbar is formed, and pbar waits in LDS during
-  // the base-field transforms, so that neither is spilled to scratch.
-  static constexpr bool PARK = !SPLIT && NW > 4;
-  // signals exchanged per LDS round of the transforms; the per-wave region
-  // also holds the partner swap of the base fields (64 x 12 doubles) and,
-  // with 4 waves, of ybar (64 x 24)
+  // Parking (half tiles, 256 registers per lane): base spectra wait in LDS
+  // while pbar is formed, and pbar waits in LDS during the base-field
+  // transforms, so that neither is spilled to scratch.
+  static constexpr bool PARK = adjoint_half<MP, SPLIT>();
+  // signals transformed together; the per-wave region also holds the partner
+  // swap of the base fields (64 x 12 doubles) and, in the 512-register form,
+  // of ybar (64 x 24)
   static constexpr int GX = PARK ? 2 : 3;
   static constexpr int RW0 = 2 * GX * Shape<MP>::WAVE_CPLX;
-  static constexpr int RWS = 64 * (NW <= 4 ? 24 : 12);
+  static constexpr int RWS = 64 * (PARK ? 12 : 24);
   static constexpr int RW = RW0 > RWS ? RW0 : RWS;
   static_assert(RW >= 2 * GX * Shape<MP>::WAVE_CPLX, "exchange region too small");
   // nodal staging: two alternating chunk buffers of the base field(s)
@@ -71,17 +78,16 @@ struct AdjLds {
   // entries of one weight and reads 16 consecutive entries of each of 4
   // weights SK apart; the 16-double pad puts those groups in different bank
   // halves.  (By local node, entry-major, each item reads all 18 weights of
-  // its 7 entries, six times the LDS reads: 11.18 against 10.93 ms for the
-  // 7-wave form at M = 64, and slower on 4 waves too.)
-  static constexpr int RPL = 7 * LY::E * (MP / 4);
+  // its 7 entries, six times the LDS reads.)
+  static constexpr int RPL = point_groups<MP, LY::E>() * 64;   // points x L
   static constexpr int SK = RPL + 16;
   static constexpr int RED = SK * AdjRed<SPLIT>::K;
   // the reduction area aliases the staging and wave regions (used after them)
   static constexpr int BIGD = (NODAL + NW * RW > RED) ? NODAL + NW * RW : RED;
   // parked doubles per lane: PK1 in the staging area (idle once the base
   // fields are interpolated; slot f of lane t at f * NT + t), PK2 past BIGD
-  // in what is left of the 160 KB
-  static constexpr int LDS_DOUBLES = 160 * 1024 / 8;
+  // in what is left of the work-group's share of the 160 KB
+  static constexpr int LDS_DOUBLES = (PARK ? 80 : 160) * 1024 / 8;
   static constexpr int PK1 = PARK ? NODAL / NT : 0;
   static constexpr int PK2 = PARK ? (LDS_DOUBLES - 2 * LY::BIG - BIGD) / NT : 0;
   static constexpr int PK = PK1 + PK2;
@@ -105,8 +111,9 @@ SFX_DEV double& park_slot(double* big, int f, int t) {
 // that it fits the 256-register form (its wave region holds 12 doubles per
 // lane).  Loading the partner modes as well would double the load
 // instructions, each of which touches 16 cache lines: the work-group's
-// loads queue in the vector memory path (adjoint at M = 64: 10.93 ms with
-// own and partner loads two slots at a time, 10.56 ms with SWAP2).
+// loads queue in the vector memory path (3.5 % of the adjoint at M = 64).
+// Issued a chunk of base fields earlier they take longer, not less (9.36
+// against 9.20 ms).
 template <int MP, bool SWAP2>
 SFX_DEV void load_ybar(const AdjArgs& A, int64_t p, bool valid, int pt, int l, double* xf,
                        double2 (&Z)[2][4], double2 (&B)[2][4]) {
@@ -232,12 +239,13 @@ SFX_DEV void load_ybar(const AdjArgs& A, int64_t p, bool valid, int pt, int l, d
 template <int MP, bool SPLIT, int NW>
 SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem) {
   using S = Shape<MP>;
-  using LY = GaussLds<MP, NW>;
   using AL = AdjLds<MP, SPLIT, NW>;
+  using LY = typename AL::LY;
   constexpr int KR = AdjRed<SPLIT>::K;
   (void)KR;   // bounds checks only
   const GaussArgs& a = A.g;
-  constexpr int L = S::L, PW = S::PW, E = LY::E, N = S::N, NG = groups_per_wave(NW);
+  constexpr int L = S::L, PW = S::PW, E = LY::E, N = S::N;
+  constexpr int NGR = point_groups<MP, E>(), NG = groups_per_wave<MP, E, NW>();
   constexpr int GX = AL::GX;
   constexpr int NT = 64 * NW;
   const int wave = tid >> 6, lane = tid & 63;
@@ -249,19 +257,19 @@ SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem)
   double2* geo = smem + LY::GEO;
   const int64_t e0 = bid * E;
   // the first chunk of the base fields leaves with the tables' loads
-  NodalSlots<MP, NW> slots;
-  NodalFetch<6, MP, NW> fa, fb;
+  NodalSlots<MP, NW, E> slots;
+  NodalFetch<6, MP, NW, E> fa, fb;
   auto fetch = [&](int c) {
-    nodal_fetch<6, MP, NW>(a, a.U, a.nU, c, tid, slots, fa);
-    if (SPLIT) nodal_fetch<6, MP, NW>(a, A.UB, A.nUB, c, tid, slots, fb);
+    nodal_fetch<6, MP, NW, E>(a, a.U, a.nU, c, tid, slots, fa);
+    if (SPLIT) nodal_fetch<6, MP, NW, E>(a, A.UB, A.nUB, c, tid, slots, fb);
   };
-  nodal_slots<MP, NW>(a, e0, tid, slots);
-  gauss_prologue<MP, NW>(a, tid, e0, smem, [&] { fetch(0); });
+  nodal_slots(a, e0, tid, slots);
+  gauss_prologue<MP, NW, E>(a, tid, e0, smem, [&] { fetch(0); });
   SFX_SYNC();
   const double2* wN = tw;
   const double2* wMP = tw + 3 * MP;
 
-  // ---- this lane's Gauss point in each of the wave's groups (group wave + 4 gi)
+  // ---- this lane's Gauss point in each of the wave's groups (group wave + NW gi)
   GaussGeom g[NG];
   bool has[NG], valid[NG];
   int el[NG];
@@ -269,11 +277,12 @@ SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem)
 #pragma unroll
   for (int gi = 0; gi < NG; ++gi) {
     const int grp = wave + NW * gi;
-    has[gi] = grp < GAUSS_GROUPS;
+    has[gi] = grp < NGR;
     const int lp = (has[gi] ? grp : 0) * PW + pt;
-    el[gi] = lp / 7;
+    const bool in = lp < 7 * E;   // the last group of half tiles is half past their elements
+    el[gi] = in ? lp / 7 : 0;
     p[gi] = e0 * 7 + lp;
-    valid[gi] = has[gi] && (e0 + el[gi]) < a.me;
+    valid[gi] = has[gi] && in && (e0 + el[gi]) < a.me;
     gauss_geom(geo + 6 * el[gi], tab, valid[gi] ? lp % 7 : 0, g[gi]);
   }
   double* big = smd + 2 * LY::BIG;
@@ -294,8 +303,8 @@ SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem)
       // chunk c into buffer c % 2 (chunk c - 2 there was interpolated by
       // every wave before the last barrier), fetch chunk c + 1, one barrier
       double* nodA = big + (c & 1) * (SPLIT ? 2 : 1) * LY::NOD6;
-      nodal_store<6, MP, NW>(fa, tid, nodA, LY::ROW6);
-      if (SPLIT) nodal_store<6, MP, NW>(fb, tid, nodA + LY::NOD6, LY::ROW6);
+      nodal_store<6, MP, NW, E>(fa, tid, nodA, LY::ROW6);
+      if (SPLIT) nodal_store<6, MP, NW, E>(fb, tid, nodA + LY::NOD6, LY::ROW6);
       if (c < 3) fetch(c + 1);
       SFX_SYNC();
       const int m = c * L + l;
@@ -430,7 +439,7 @@ SFX_DEV void adjoint_body(const AdjArgs& A, int tid, int64_t bid, double2* smem)
 #pragma unroll
   for (int gi = 0; gi < NG; ++gi) {
     const int lpg = (wave + NW * gi) * PW + pt;
-    int elg = lpg / 7;
+    int elg = lpg < 7 * E ? lpg / 7 : 0;
     SFX_OPAQUE(elg);
     gauss_geom(geo + 6 * elg, tab, valid[gi] ? lpg % 7 : 0, gr[gi]);
   }

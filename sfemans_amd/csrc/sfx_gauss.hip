@@ -54,20 +54,25 @@ static hipError_t launch_v(const GaussArgs& a, hipStream_t st) {
 
 // The fused nodal -> assembly element sums (RHS form of the body):
 // cross-curl -> rhs_3x3, u.grad c -> qs_00_gauss.
-template <int MP, int V, int NW = gauss_waves<MP, V>()>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NW), waves_per_simd(NW))))
+template <int MP, int V>
+constexpr int gauss_rhs_occupancy() { return gauss_rhs_half<MP>() ? 2 : waves_per_simd(gauss_rhs_waves<MP, V>()); }
+
+template <int MP, int V, int NW = gauss_rhs_waves<MP, V>()>
+__global__ void __launch_bounds__(64 * NW)
+__attribute__((amdgpu_waves_per_eu(gauss_rhs_occupancy<MP, V>(), gauss_rhs_occupancy<MP, V>())))
 gauss_rhs_kernel(GaussArgs a) {
   extern __shared__ double2 smem[];
-  gauss_body<MP, V, NW, false, true>(a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x), smem);
+  gauss_body<MP, V, NW, false, true, false, gauss_rhs_elems<MP>()>(a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x),
+                                                                  smem);
 }
 
 template <int MP, int V>
 static hipError_t launch_rhs_mp(const GaussArgs& a, hipStream_t st) {
-  constexpr int NW = gauss_waves<MP, V>();
-  constexpr int E = GaussLds<MP, NW>::E;
+  constexpr int NW = gauss_rhs_waves<MP, V>();
+  constexpr int E = gauss_rhs_elems<MP>();
   const int64_t nblk = (a.me + E - 1) / E;
   if (nblk == 0) return hipSuccess;
-  const size_t shmem = (size_t)GaussCfg<MP, V, NW>::LY::TOTAL * sizeof(double2);
+  const size_t shmem = (size_t)GaussCfg<MP, V, NW, false, E>::LY::TOTAL * sizeof(double2);
   hipLaunchKernelGGL((gauss_rhs_kernel<MP, V>), dim3((unsigned)nblk), dim3(64 * NW), shmem, st, a);
   return hipGetLastError();
 }

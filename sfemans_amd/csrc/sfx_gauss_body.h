@@ -15,7 +15,8 @@
 //                  subroutine_ns_with_velocity.F90:227, 246-248, in one launch; and
 //                  the tangents (curl U) x d + (curl d) x U (+ Lorentz terms).
 //
-// Work decomposition (point tiles aside, see gauss_point_tiles): a work-group
+// Work decomposition (point and half tiles aside, see gauss_point_tiles and
+// gauss_rhs_half): a work-group
 // owns E = 256/MP consecutive elements, i.e.
 // 7E consecutive Gauss points (index (m-1)*7 + l), cut into 7 groups of
 // PW = 256/MP points (L = MP/4 lanes each, see sfx_engine.h).  The work-group
@@ -44,21 +45,44 @@ template <> struct GVT<GV_PAIRS>      { static constexpr int NSIG = 3, NOUT = 3,
 template <> struct GVT<GV_CURL_CROSS> { static constexpr int NSIG = 3, NOUT = 3, MAXP = 1; };
 template <> struct GVT<GV_UGRADC>     { static constexpr int NSIG = 4, NOUT = 1, MAXP = 1; };
 
-constexpr int GAUSS_GROUPS = 7;   // point groups per work-group
 constexpr int GAUSS_WAVES = 4;    // default wave count (batched launches)
 // Waves per work-group of the fused kernel for variant V at size MP.  With 7
 // waves a wave holds one group and a CU runs two waves per SIMD (256
 // registers each), which hides more latency; with 4 waves a wave holds two
 // groups in 512 registers at one wave per SIMD.  7 where measured faster:
-// u.grad c; the cross-curl up to MP = 128 (at M = 128, 200,704 triangles,
-// the fused right-hand side 19.1 -> 17.8 ms and the Gauss output 16.4 ->
-// 16.2 ms against 4 waves, despite 152 bytes per lane of spill); the
-// single-pass (curl a) x b up to MP = 64.  4 elsewhere.
+// u.grad c; the cross-curl up to MP = 128 (Gauss output at M = 128, 200,704
+// triangles, 16.4 -> 16.2 ms against 4 waves); the single-pass (curl a) x b up
+// to MP = 64.  4 elsewhere.
 template <int MP, int V>
 constexpr int gauss_waves() {
   return (V == GV_UGRADC || (V == GV_CROSS_CURL && MP <= 128) || (V == GV_CURL_CROSS && MP <= 64)) ? 7 : 4;
 }
-constexpr int groups_per_wave(int nw) { return (GAUSS_GROUPS + nw - 1) / nw; }
+// Point groups (of PW = 256/MP points) of E elements, and of a wave of NW.
+template <int MP, int E>
+constexpr int point_groups() { return (7 * E + 256 / MP - 1) / (256 / MP); }
+template <int MP, int E, int NW>
+constexpr int groups_per_wave() { return (point_groups<MP, E>() + NW - 1) / NW; }
+// Elements per work-group: 256/MP (7 groups).
+template <int MP>
+constexpr int gauss_elems() { return 256 / MP; }
+
+// Half tiles (the element sums up to MP = 128): a work-group of 4 waves takes
+// half the elements, 3.5 groups of points, in 256 registers per lane and at
+// most half the LDS, so that two work-groups share a CU.  The points per wave
+// are those of 7 waves with 7 groups (3.5 of 4 groups against 7 of 8 wave
+// slots), but a CU no longer stops as a whole at each barrier: a wave of the
+// 7-wave form at M = 100 spent 20,000 of 76,000 cycles waiting in the element
+// sums and 10,000 for its first chunk.  Fused right-hand side, half against whole
+// tiles: 1.23 / 1.40 ms at MP = 4 (767,000 triangles), 1.10 / 1.26 at 8, 1.14 /
+// 1.28 at 16, 1.26 / 1.42 at 32, 1.31 / 1.50 at 64, 1.49 / 1.80 at 128 (23,700);
+// u.grad c 1.25 / 1.46, 1.15 / 1.32, 1.27 / 1.47, 1.32 / 1.58, 1.48 / 1.72 and
+// 1.80 / 2.05; no slower where few work-groups run.
+template <int MP>
+constexpr bool gauss_rhs_half() { return MP <= 128; }
+template <int MP, int V>
+constexpr int gauss_rhs_waves() { return gauss_rhs_half<MP>() ? 4 : gauss_waves<MP, V>(); }
+template <int MP>
+constexpr int gauss_rhs_elems() { return gauss_rhs_half<MP>() ? 128 / MP : gauss_elems<MP>(); }
 
 // Point tiles (the plain Gauss-point output of the cross-curl at 16 <= MP
 // <= 64): a work-group of GAUSS_PT_WAVES waves takes GAUSS_PT_WAVES * PW
@@ -86,9 +110,9 @@ constexpr int waves_per_simd(int nw) { return nw > 4 ? 2 : 1; }
 // LDS layout (double2 units) of the fused kernel with NW waves.  The nodal
 // staging holds NCH chunks (1: one chunk at a time; 4: all modes at once)
 // of a 6-column field and a second field of NCB columns (6, 2 or 0).
-template <int MP, int NW = GAUSS_WAVES, int NCH = 1, int NCB = 6>
+template <int MP, int NW = GAUSS_WAVES, int NCH = 1, int NCB = 6, int EL = gauss_elems<MP>()>
 struct GaussLds {
-  static constexpr int E = 256 / MP;                    // elements per work-group
+  static constexpr int E = EL;                          // elements per work-group
   static constexpr int L = MP / 4;
   static constexpr int TW = 0;                          // twiddles, 4 MP
   static constexpr int TAB = 4 * MP;                    // ww(6,7), dd(2,6,7): 126 doubles
@@ -123,14 +147,14 @@ constexpr int GAUSS_LDS_BYTES = 160 * 1024;
 // STAGE_ALL (used by the batched launch, measured faster there) all four
 // chunks are staged at once where that fits in LDS and the variant makes a
 // single pass over its fields: one barrier, every load in flight together.
-template <int MP, int V, int NW, bool STAGE_ALL = false>
+template <int MP, int V, int NW, bool STAGE_ALL = false, int E = gauss_elems<MP>()>
 struct GaussCfg {
   static constexpr int NCB = (V == GV_UGRADC) ? 2 : ((V == GV_PAIRS || V == GV_CURL_CROSS) ? 6 : 0);
   static constexpr bool ALL =
-      STAGE_ALL && V != GV_PAIRS && GaussLds<MP, NW, 4, NCB>::TOTAL * 16 <= GAUSS_LDS_BYTES;
+      STAGE_ALL && V != GV_PAIRS && GaussLds<MP, NW, 4, NCB, E>::TOTAL * 16 <= GAUSS_LDS_BYTES;
   // chunk buffers when not staging all at once: two where they fit
-  static constexpr int NBUF = GaussLds<MP, NW, 2, NCB>::TOTAL * 16 <= GAUSS_LDS_BYTES ? 2 : 1;
-  using LY = GaussLds<MP, NW, ALL ? 4 : NBUF, NCB>;
+  static constexpr int NBUF = GaussLds<MP, NW, 2, NCB, E>::TOTAL * 16 <= GAUSS_LDS_BYTES ? 2 : 1;
+  using LY = GaussLds<MP, NW, ALL ? 4 : NBUF, NCB, E>;
   static_assert(LY::TOTAL * 16 <= GAUSS_LDS_BYTES, "LDS of the work-group");
 };
 
@@ -258,16 +282,16 @@ SFX_DEV T pick(const T (&v)[N], int i) {
 // strides, at 200,704 triangles, M = 64: 4453 -> 3820 vector instructions per
 // wave, forward term 4.22 -> 3.81 ms; tangent at 99,856 triangles, M = 32, 3.57
 // -> 3.25 ms.
-template <int MP, int NW>
+template <int MP, int NW, int E = gauss_elems<MP>()>
 struct NodalSlots {
-  static constexpr int S = GaussLds<MP>::E * 6, NT = 64 * NW;
+  static constexpr int S = E * 6, NT = 64 * NW;
   static constexpr int SI = (S + NT - 1) / NT;          // slots per thread
   static constexpr int R = SI > 1 ? 1 : NT / S;         // threads per slot
   int node[SI];                                         // node (from 0) of the thread's slots
 };
-template <int NC, int MP, int NW>
+template <int NC, int MP, int NW, int E = gauss_elems<MP>()>
 struct NodalFetch {
-  using SL = NodalSlots<MP, NW>;
+  using SL = NodalSlots<MP, NW, E>;
   static constexpr int S = SL::S, NT = SL::NT, SI = SL::SI, R = SL::R;
   static constexpr int Q = NC * (MP / 4);
   static constexpr int IT = (Q + R - 1) / R;
@@ -275,9 +299,9 @@ struct NodalFetch {
 };
 
 // The thread's slots of the E elements from e0 on (node 0 past the last element).
-template <int MP, int NW>
-SFX_DEV void nodal_slots(const GaussArgs& a, int64_t e0, int tid, NodalSlots<MP, NW>& f) {
-  using F = NodalSlots<MP, NW>;
+template <int MP, int NW, int E>
+SFX_DEV void nodal_slots(const GaussArgs& a, int64_t e0, int tid, NodalSlots<MP, NW, E>& f) {
+  using F = NodalSlots<MP, NW, E>;
 #pragma unroll
   for (int si = 0; si < F::SI; ++si) {
     const int t = tid + si * F::NT;
@@ -292,10 +316,10 @@ SFX_DEV void nodal_slots(const GaussArgs& a, int64_t e0, int tid, NodalSlots<MP,
 // Issue the loads of chunk c into registers: unconditional (planes past the
 // last mode read the slot's first value, which no interpolation uses), so that
 // they all issue back to back and overlap other work.
-template <int NC, int MP, int NW>
+template <int NC, int MP, int NW, int E>
 SFX_DEV void nodal_fetch(const GaussArgs& a, const double* X, int64_t nX, int c, int tid,
-                         const NodalSlots<MP, NW>& sl, NodalFetch<NC, MP, NW>& f) {
-  using F = NodalFetch<NC, MP, NW>;
+                         const NodalSlots<MP, NW, E>& sl, NodalFetch<NC, MP, NW, E>& f) {
+  using F = NodalFetch<NC, MP, NW, E>;
 #pragma unroll
   for (int si = 0; si < F::SI; ++si) {
     const int t = tid + si * F::NT;
@@ -314,9 +338,9 @@ SFX_DEV void nodal_fetch(const GaussArgs& a, const double* X, int64_t nX, int c,
 }
 
 // Store a fetched chunk to LDS.
-template <int NC, int MP, int NW>
-SFX_DEV void nodal_store(const NodalFetch<NC, MP, NW>& f, int tid, double* nod, int row) {
-  using F = NodalFetch<NC, MP, NW>;
+template <int NC, int MP, int NW, int E>
+SFX_DEV void nodal_store(const NodalFetch<NC, MP, NW, E>& f, int tid, double* nod, int row) {
+  using F = NodalFetch<NC, MP, NW, E>;
 #pragma unroll
   for (int si = 0; si < F::SI; ++si) {
     const int t = tid + si * F::NT;
@@ -404,10 +428,10 @@ SFX_DEV void pass_fields(const GaussArgs& a, const double* nodA, const double* n
 // numbers, node coordinates and node numbers of the E elements.  All loads
 // issue together (clamped indices), then what `issue` loads for the caller,
 // then the LDS stores.
-template <int MP, int NW, class Issue>
+template <int MP, int NW, int E, class Issue>
 SFX_DEV void gauss_prologue(const GaussArgs& a, int tid, int64_t e0, double2* smem, const Issue& issue) {
-  using LY = GaussLds<MP, NW>;
-  constexpr int E = LY::E, NT = 64 * NW;
+  using LY = GaussLds<MP, NW, 1, 6, E>;
+  constexpr int NT = 64 * NW;
   double* smd = reinterpret_cast<double*>(smem);
   double2* tw = smem + LY::TW;
   double* tab = smd + 2 * LY::TAB;
@@ -470,12 +494,13 @@ SFX_DEV void gauss_prologue(const GaussArgs& a, int tid, int64_t e0, double2* sm
 // (one group per wave) instead of E whole elements: the points of at most
 // E elements, the first one e0 = p0 / 7, all of them staged.  For the
 // Gauss-point output only (the element sums of RHS need whole elements).
-template <int MP, int V, int NW, bool STAGE_ALL = false, bool RHS = false, bool PT = false>
+template <int MP, int V, int NW, bool STAGE_ALL = false, bool RHS = false, bool PT = false, int E = gauss_elems<MP>()>
 SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem) {
   using S = Shape<MP>;
-  using LY = typename GaussCfg<MP, V, NW, STAGE_ALL>::LY;
-  constexpr bool ALL = GaussCfg<MP, V, NW, STAGE_ALL>::ALL;
-  constexpr int L = S::L, PW = S::PW, E = LY::E, NG = PT ? 1 : groups_per_wave(NW);
+  using CFG = GaussCfg<MP, V, NW, STAGE_ALL, E>;
+  using LY = typename CFG::LY;
+  constexpr bool ALL = CFG::ALL;
+  constexpr int L = S::L, PW = S::PW, NGR = point_groups<MP, E>(), NG = PT ? 1 : groups_per_wave<MP, E, NW>();
   static_assert(!PT || (!RHS && !STAGE_ALL && (NW * PW + 5) / 7 + 1 <= E), "point tiles: Gauss output only");
   constexpr int NSIG = GVT<V>::NSIG, NO = GVT<V>::NOUT;
   // Outputs staged in LDS and stored in whole runs of the work-group's points
@@ -508,12 +533,13 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
 #pragma unroll
   for (int gi = 0; gi < NG; ++gi) {
     const int grp = wave + NW * gi;
-    has[gi] = PT || grp < GAUSS_GROUPS;
+    has[gi] = PT || grp < NGR;
     const int lp = (has[gi] ? grp : 0) * PW + pt;    // local point
     const int64_t pg = p0 + lp;
-    el[gi] = (int)(pg / 7 - e0);
+    // (the last group of half tiles is half past their elements)
+    valid[gi] = has[gi] && pg < 7 * a.me && (PT || lp < 7 * E);
+    el[gi] = PT || lp < 7 * E ? (int)(pg / 7 - e0) : 0;
     p[gi] = pg;
-    valid[gi] = has[gi] && pg < 7 * a.me;
     lq[gi] = valid[gi] ? (int)(pg % 7) : 0;
   }
 
@@ -528,20 +554,20 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
   constexpr bool EARLY = !ALL && V != GV_PAIRS;
   constexpr int NCB = (V == GV_UGRADC) ? 2 : 6;
   constexpr int DEP = ALL ? 4 : (PT || V == GV_CURL_CROSS) ? 2 : 1;   // chunks in registers
-  NodalSlots<MP, NW> slots;
-  NodalFetch<6, MP, NW> fa[DEP];
-  NodalFetch<NCB, MP, NW> fb[DEP];
+  NodalSlots<MP, NW, E> slots;
+  NodalFetch<6, MP, NW, E> fa[DEP];
+  NodalFetch<NCB, MP, NW, E> fb[DEP];
   auto fetch = [&](const double* XA, int64_t nXA, const double* XB, int64_t nXB, bool useB, int c) {
-    nodal_fetch<6, MP, NW>(a, XA, nXA, c, tid, slots, fa[c % DEP]);
-    if (useB) nodal_fetch<NCB, MP, NW>(a, XB, nXB, c, tid, slots, fb[c % DEP]);
+    nodal_fetch<6, MP, NW, E>(a, XA, nXA, c, tid, slots, fa[c % DEP]);
+    if (useB) nodal_fetch<NCB, MP, NW, E>(a, XB, nXB, c, tid, slots, fb[c % DEP]);
   };
   const double* XA = V == GV_CURL_CROSS ? a.pc[0] : a.U;
   const double* XB = V == GV_CURL_CROSS ? a.pv[0] : a.U2;
   int64_t nXA = V == GV_CURL_CROSS ? a.npc[0] : a.nU, nXB = V == GV_CURL_CROSS ? a.npv[0] : a.nU2;
   double coef = V == GV_CURL_CROSS ? a.coef[0] : 1.0;
   bool useB = V == GV_UGRADC || (V == GV_CURL_CROSS && XB != XA);
-  nodal_slots<MP, NW>(a, e0, tid, slots);
-  gauss_prologue<MP, NW>(a, tid, e0, smem, [&] {
+  nodal_slots(a, e0, tid, slots);
+  gauss_prologue<MP, NW, E>(a, tid, e0, smem, [&] {
 #pragma unroll
     for (int gi = 0; gi < NG; ++gi)
       hc[gi] = V == GV_UGRADC ? a.heat_capa[valid[gi] ? e0 + el[gi] : 0] : 1.0;
@@ -612,12 +638,12 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
         // every chunk at once: all loads issue back to back, one barrier
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          nodal_store<6, MP, NW>(fa[c], tid, big + c * LY::NODC, LY::ROW6);
-          if (useB) nodal_store<NCB, MP, NW>(fb[c], tid, big + c * LY::NODC + LY::NOD6, NCB == 6 ? LY::ROW6 : LY::ROW2);
+          nodal_store<6, MP, NW, E>(fa[c], tid, big + c * LY::NODC, LY::ROW6);
+          if (useB) nodal_store<NCB, MP, NW, E>(fb[c], tid, big + c * LY::NODC + LY::NOD6, NCB == 6 ? LY::ROW6 : LY::ROW2);
         }
         SFX_SYNC();
       }
-      constexpr int NBUF = GaussCfg<MP, V, NW, STAGE_ALL>::NBUF;
+      constexpr int NBUF = CFG::NBUF;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         double* nodA = big + (ALL ? c : (NBUF == 2 ? (c & 1) : 0)) * LY::NODC;
@@ -628,8 +654,8 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
           // fetching chunk c + DEP, and one barrier makes chunk c visible.  One
           // buffer: wait until every wave is done with chunk c - 1 first.
           if (NBUF == 1) SFX_SYNC();
-          nodal_store<6, MP, NW>(fa[c % DEP], tid, nodA, LY::ROW6);
-          if (useB) nodal_store<NCB, MP, NW>(fb[c % DEP], tid, nodB, NCB == 6 ? LY::ROW6 : LY::ROW2);
+          nodal_store<6, MP, NW, E>(fa[c % DEP], tid, nodA, LY::ROW6);
+          if (useB) nodal_store<NCB, MP, NW, E>(fb[c % DEP], tid, nodB, NCB == 6 ? LY::ROW6 : LY::ROW2);
           if (NBUF == 1) SFX_SYNC();
           if (c + DEP < 4) fetch(XA, nXA, XB, nXB, useB, c + DEP);
           if (NBUF == 2) SFX_SYNC();
@@ -795,7 +821,7 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
     // of the current slot; wl[lp] = wgt(e, l) of the point.  Both alias the
     // staging and wave regions, which every wave has finished with at the
     // first barrier.
-    constexpr int NPT = 7 * E;
+    constexpr int NPT = NGR * PW;   // 7 E, and the rest of the last group
     double* red = big;
     double* wl = big + NPT * L * NKR;
     static_assert(NPT * L * NKR + NPT <= LY::NODAL + NW * LY::RW, "RHS reduction area");
@@ -813,7 +839,7 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
           red[(lp * L + l) * NKR + k] = ok ? ro[gi][k][r] : 0.0;
         }
         if (r == 0 && l == 0) {
-          const int64_t wi = valid[gi] ? 7 * e0 + lp : 0;   // points past the last element read entry 0
+          const int64_t wi = valid[gi] ? 7 * e0 + lp : 0;   // points past the elements read entry 0
           SFX_CHECK("rhs wgt", wi, 7 * a.me);
           const double wv = a.wgt[wi];
           wl[lp] = valid[gi] ? wv : 0.0;

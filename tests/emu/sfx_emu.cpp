@@ -331,8 +331,8 @@ extern "C" int emu_rhs_ns(const int32_t* jj, const double* rr, int64_t me, int64
 
 template <int MP, bool SPLIT>
 static void emu_adjoint_mp(const AdjArgs& A) {
-  constexpr int NW = adjoint_waves<MP, SPLIT>();
-  constexpr int E = GaussLds<MP, NW>::E;
+  constexpr int NW = ADJOINT_WAVES;
+  constexpr int E = adjoint_elems<MP, SPLIT>();
   const int64_t nblk = (A.g.me + E - 1) / E;
   run_grid(nblk, 64 * NW, AdjLds<MP, SPLIT, NW>::TOTAL,
            [&](int t, int64_t b, double2* s) { adjoint_body<MP, SPLIT, NW>(A, t, b, s); });
@@ -893,11 +893,11 @@ extern "C" int emu_sanitizer_probe(int which, int n) {
 // vb_145/vb_236 (np, 3, M) = scale * rhs_3x3((curl u + 2 Omega) x u)
 template <int MP>
 static void emu_nl_rhs_mp(const GaussArgs& a) {
-  constexpr int NW = gauss_waves<MP, GV_CROSS_CURL>();
-  constexpr int E = GaussLds<MP, NW>::E;
+  constexpr int NW = gauss_rhs_waves<MP, GV_CROSS_CURL>();
+  constexpr int E = gauss_rhs_elems<MP>();
   const int64_t nblk = (a.me + E - 1) / E;
-  run_grid(nblk, 64 * NW, GaussCfg<MP, GV_CROSS_CURL, NW>::LY::TOTAL,
-           [&](int t, int64_t b, double2* s) { gauss_body<MP, GV_CROSS_CURL, NW, false, true>(a, t, b, s); });
+  run_grid(nblk, 64 * NW, GaussCfg<MP, GV_CROSS_CURL, NW, false, E>::LY::TOTAL,
+           [&](int t, int64_t b, double2* s) { gauss_body<MP, GV_CROSS_CURL, NW, false, true, false, E>(a, t, b, s); });
 }
 
 extern "C" int emu_nl_rhs(const int32_t* jj, const double* rr, int64_t me, int64_t np, const double* U,
@@ -949,11 +949,11 @@ extern "C" int emu_nl_rhs(const int32_t* jj, const double* rr, int64_t me, int64
 // vect (np, 2, M) = scale * qs_00_gauss(hc, ff, (hc grad c).u + (div u)(hc c))
 template <int MP>
 static void emu_nl_qs00_mp(const GaussArgs& a) {
-  constexpr int NW = gauss_waves<MP, GV_UGRADC>();
-  constexpr int E = GaussLds<MP, NW>::E;
+  constexpr int NW = gauss_rhs_waves<MP, GV_UGRADC>();
+  constexpr int E = gauss_rhs_elems<MP>();
   const int64_t nblk = (a.me + E - 1) / E;
-  run_grid(nblk, 64 * NW, GaussCfg<MP, GV_UGRADC, NW>::LY::TOTAL,
-           [&](int t, int64_t b, double2* s) { gauss_body<MP, GV_UGRADC, NW, false, true>(a, t, b, s); });
+  run_grid(nblk, 64 * NW, GaussCfg<MP, GV_UGRADC, NW, false, E>::LY::TOTAL,
+           [&](int t, int64_t b, double2* s) { gauss_body<MP, GV_UGRADC, NW, false, true, false, E>(a, t, b, s); });
 }
 
 extern "C" int emu_nl_qs00(const int32_t* jj, const double* rr, int64_t me, int64_t np, const double* U,
