@@ -17,23 +17,42 @@ template <int MP, int V>
 __global__ void __launch_bounds__(64 * GAUSS_PT_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gauss_pt_kernel(GaussArgs a) {
   extern __shared__ double2 smem[];
-  gauss_body<MP, V, GAUSS_PT_WAVES, false, false, true>(a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x), smem);
+  gauss_body<MP, V, GAUSS_PT_WAVES, false, false, true, gauss_pt_elems<MP>()>(
+      a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x), smem);
+}
+
+template <int MP, int V>
+static hipError_t launch_whole(const GaussArgs& a, hipStream_t st) {
+  constexpr int NW = gauss_waves<MP, V>();
+  const int64_t nblk = gauss_whole_blocks<MP>(a.me);
+  if (nblk == 0) return hipSuccess;
+  const size_t shmem = (size_t)GaussCfg<MP, V, NW>::LY::TOTAL * sizeof(double2);
+  hipLaunchKernelGGL((gauss_kernel<MP, V>), dim3((unsigned)nblk), dim3(64 * NW), shmem, st, a);
+  return hipGetLastError();
+}
+
+// Half tiles (see gauss_half): 4 waves, two per SIMD.
+template <int MP, int V>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) gauss_half_kernel(GaussArgs a) {
+  extern __shared__ double2 smem[];
+  gauss_body<MP, V, 4, false, false, false, 128 / MP>(a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x), smem);
 }
 
 template <int MP, int V>
 static hipError_t launch_mp(const GaussArgs& a, hipStream_t st) {
+  if constexpr (gauss_one_round<MP, V>()) {
+    if (gauss_take_whole<MP, V>(a.me)) return launch_whole<MP, V>(a, st);
+  }
+  const int64_t nblk = gauss_blocks<MP, V>(a.me);
+  if (nblk == 0) return hipSuccess;
   if constexpr (gauss_point_tiles<MP, V>()) {
-    constexpr int NW = GAUSS_PT_WAVES;
-    const int64_t nblk = gauss_blocks<MP, V, NW>(a.me);
-    if (nblk == 0) return hipSuccess;
-    const size_t shmem = (size_t)GaussCfg<MP, V, NW>::LY::TOTAL * sizeof(double2);
-    hipLaunchKernelGGL((gauss_pt_kernel<MP, V>), dim3((unsigned)nblk), dim3(64 * NW), shmem, st, a);
+    const size_t shmem = (size_t)GaussPtCfg<MP, V>::LY::TOTAL * sizeof(double2);
+    hipLaunchKernelGGL((gauss_pt_kernel<MP, V>), dim3((unsigned)nblk), dim3(64 * GAUSS_PT_WAVES), shmem, st, a);
+  } else if constexpr (gauss_half<MP, V>()) {
+    const size_t shmem = (size_t)GaussHalfCfg<MP, V>::LY::TOTAL * sizeof(double2);
+    hipLaunchKernelGGL((gauss_half_kernel<MP, V>), dim3((unsigned)nblk), dim3(256), shmem, st, a);
   } else {
-    constexpr int NW = gauss_waves<MP, V>();
-    const int64_t nblk = gauss_blocks<MP, V, NW>(a.me);
-    if (nblk == 0) return hipSuccess;
-    const size_t shmem = (size_t)GaussCfg<MP, V, NW>::LY::TOTAL * sizeof(double2);
-    hipLaunchKernelGGL((gauss_kernel<MP, V>), dim3((unsigned)nblk), dim3(64 * NW), shmem, st, a);
+    return launch_whole<MP, V>(a, st);
   }
   return hipGetLastError();
 }
@@ -72,7 +91,7 @@ static hipError_t launch_rhs_mp(const GaussArgs& a, hipStream_t st) {
   constexpr int E = gauss_rhs_elems<MP>();
   const int64_t nblk = (a.me + E - 1) / E;
   if (nblk == 0) return hipSuccess;
-  const size_t shmem = (size_t)GaussCfg<MP, V, NW, false, E>::LY::TOTAL * sizeof(double2);
+  const size_t shmem = (size_t)GaussRhsCfg<MP, V>::LY::TOTAL * sizeof(double2);
   hipLaunchKernelGGL((gauss_rhs_kernel<MP, V>), dim3((unsigned)nblk), dim3(64 * NW), shmem, st, a);
   return hipGetLastError();
 }

@@ -30,6 +30,8 @@
 // isoparametric Jacobian, exact for curved P2 elements), radius from the six
 // nodes as the reference.
 #pragma once
+#include <type_traits>
+
 #include "sfx_engine.h"
 #include "sfx_fftprod_body.h"
 #include "sfx_geom.h"
@@ -50,13 +52,10 @@ constexpr int GAUSS_WAVES = 4;    // default wave count (batched launches)
 // waves a wave holds one group and a CU runs two waves per SIMD (256
 // registers each), which hides more latency; with 4 waves a wave holds two
 // groups in 512 registers at one wave per SIMD.  7 where measured faster:
-// u.grad c; the cross-curl up to MP = 128 (Gauss output at M = 128, 200,704
-// triangles, 16.4 -> 16.2 ms against 4 waves); the single-pass (curl a) x b up
-// to MP = 64.  4 elsewhere.
+// u.grad c and the cross-curl up to MP = 128 (Gauss output at M = 128, 200,704
+// triangles, 16.4 -> 16.2 ms against 4 waves).  4 elsewhere.
 template <int MP, int V>
-constexpr int gauss_waves() {
-  return (V == GV_UGRADC || (V == GV_CROSS_CURL && MP <= 128) || (V == GV_CURL_CROSS && MP <= 64)) ? 7 : 4;
-}
+constexpr int gauss_waves() { return (V == GV_UGRADC || (V == GV_CROSS_CURL && MP <= 128)) ? 7 : 4; }
 // Point groups (of PW = 256/MP points) of E elements, and of a wave of NW.
 template <int MP, int E>
 constexpr int point_groups() { return (7 * E + 256 / MP - 1) / (256 / MP); }
@@ -84,26 +83,53 @@ constexpr int gauss_rhs_waves() { return gauss_rhs_half<MP>() ? 4 : gauss_waves<
 template <int MP>
 constexpr int gauss_rhs_elems() { return gauss_rhs_half<MP>() ? 128 / MP : gauss_elems<MP>(); }
 
-// Point tiles (the plain Gauss-point output of the cross-curl at 16 <= MP
-// <= 64): a work-group of GAUSS_PT_WAVES waves takes GAUSS_PT_WAVES * PW
-// consecutive Gauss points instead of E whole elements.  With 16 points at
-// MP = 64 each plane of the output gets one whole 128-byte line per
+// Point tiles (the Gauss-point output of the cross-curl up to MP = 128, and of
+// the other single passes at MP = 4): a work-group of GAUSS_PT_WAVES waves takes
+// GAUSS_PT_WAVES * PW consecutive Gauss points instead of whole elements.  With
+// 16 points at MP = 64 each plane of the output gets one whole 128-byte line per
 // work-group (28 points of whole elements straddle lines, and the partial
-// lines cost 1.7x the output bytes of HBM writes), and the 76-77 KB of LDS
-// let two work-groups share a CU (256 registers per lane, two waves per
-// SIMD).  The outputs leave through LDS, each store instruction writing 4
-// planes x 16 points (a lane's own stores touch 16 planes x 4 points, 16
-// cache lines).  Measured at 200,704 triangles: 5.72 -> 5.56 ms at M = 64,
-// 2.87 -> 2.64 ms at M = 32, 1.06 -> 1.05 ms at M = 16; staged stores 5.56
-// -> 5.28 and 2.66 -> 2.52 ms; output bit for bit the same.
+// lines cost 1.7x the output bytes of HBM writes), and half the LDS lets two
+// work-groups share a CU (256 registers per lane, two waves per SIMD).  The
+// outputs leave through LDS, each store instruction writing 4 planes x 16
+// points (a lane's own stores touch 16 planes x 4 points, 16 cache lines).
+// Against 7 waves on whole elements: 0.33 / 0.36 ms at MP = 4, 0.36 / 0.40 at 8,
+// 0.55 / 0.73 at 128 (7,744 triangles); u.grad c 0.30 / 0.44 and tangent 0.99 /
+// 1.31 at MP = 4.  From MP = 8 on these two would stage both fields of the
+// points' elements with 30 to 60 spilled registers per lane; half tiles
+// (gauss_half) are faster for them.
 constexpr int GAUSS_PT_WAVES = 4;
 template <int MP, int V>
-constexpr bool gauss_point_tiles() { return V == GV_CROSS_CURL && MP >= 16 && MP <= 64; }
-// Work-groups of the launch over me elements.
-template <int MP, int V, int NW>
+constexpr bool gauss_point_tiles() { return V == GV_CROSS_CURL ? MP <= 128 : V != GV_PAIRS && MP == 4; }
+// Elements that the points of a tile can touch.
+template <int MP>
+constexpr int gauss_pt_elems() { return (GAUSS_PT_WAVES * (256 / MP) + 5) / 7 + 1; }
+// Half tiles (see gauss_rhs_half) of the Gauss-point output: u.grad c 0.37 / 0.39
+// ms at MP = 8 against 7 waves on whole elements, 0.44 / 0.48 at 32, 0.49 / 0.54
+// at 64, 0.59 / 0.70 at 128; tangent 1.09 / 1.32, 1.25 / 1.57 and 1.42 / 1.79 at
+// 8, 32 and 64 (at 128 its two fields take more than half the LDS).
+template <int MP, int V>
+constexpr bool gauss_half() { return MP >= 8 && ((V == GV_CURL_CROSS && MP <= 64) || (V == GV_UGRADC && MP <= 128)); }
+// Work-groups of the launch over me elements: tiles of `pts` points, of whole
+// tiles' elements, and of the form that a variant takes.
+constexpr int64_t gauss_pt_blocks(int64_t me, int pts) { return (7 * me + pts - 1) / pts; }
+template <int MP>
+constexpr int64_t gauss_whole_blocks(int64_t me) { return (me + gauss_elems<MP>() - 1) / gauss_elems<MP>(); }
+template <int MP, int V>
 constexpr int64_t gauss_blocks(int64_t me) {
-  return gauss_point_tiles<MP, V>() ? (7 * me + NW * (64 / (MP / 4)) - 1) / (NW * (64 / (MP / 4)))
-                                    : (me + 256 / MP - 1) / (256 / MP);
+  if (gauss_point_tiles<MP, V>()) return gauss_pt_blocks(me, GAUSS_PT_WAVES * (256 / MP));
+  return gauss_half<MP, V>() ? (me + 128 / MP - 1) / (128 / MP) : gauss_whole_blocks<MP>(me);
+}
+// Whole elements all the same where they are one round of a work-group per CU
+// (256 of them) and the point tiles would put two on some: cross-curl at MP = 8
+// 17.7 against 18.7 us with 200 whole tiles, 15.9 against 17.0 at MP = 4 and 28.7
+// against 30.0 at 128; but 15.2 against 11.5 us with 60, and 31.1 against 26.9
+// with 400.  (At 16 <= MP <= 64 the whole tiles have no instance of their own.)
+constexpr int64_t GAUSS_CUS = 256;
+template <int MP, int V>
+constexpr bool gauss_one_round() { return V == GV_CROSS_CURL && (MP < 16 || MP == 128); }
+template <int MP, int V>
+constexpr bool gauss_take_whole(int64_t me) {
+  return gauss_one_round<MP, V>() && gauss_whole_blocks<MP>(me) <= GAUSS_CUS && gauss_blocks<MP, V>(me) > GAUSS_CUS;
 }
 constexpr int waves_per_simd(int nw) { return nw > 4 ? 2 : 1; }
 
@@ -122,8 +148,9 @@ struct GaussLds {
   static constexpr int BIG = NID + (E * 6 + 3) / 4;
   // doubles per node slot, 6 columns: 16-byte reads of the modes of one element
   // (48 bytes apart) and of the next one (6 rows on) then miss each other's banks;
-  // shorter rows at small MP, whose many elements fill the LDS
-  static constexpr int ROW6 = L * 6 + (L >= 8 ? 6 : 2);
+  // shorter rows at small MP, whose many elements fill the LDS, and where a
+  // point's lanes fill a 32-lane group (two buffers then fit in half the LDS)
+  static constexpr int ROW6 = L * 6 + (L >= 8 && L < 32 ? 6 : 2);
   static constexpr int ROW2 = L * 2 + 2;                // doubles per node slot, 2 columns
   static constexpr int NOD6 = E * 6 * ROW6;             // doubles of one staged 6-column field
   static constexpr int NOD2 = E * 6 * ROW2;
@@ -147,16 +174,26 @@ constexpr int GAUSS_LDS_BYTES = 160 * 1024;
 // STAGE_ALL (used by the batched launch, measured faster there) all four
 // chunks are staged at once where that fits in LDS and the variant makes a
 // single pass over its fields: one barrier, every load in flight together.
-template <int MP, int V, int NW, bool STAGE_ALL = false, int E = gauss_elems<MP>()>
+template <int MP, int V, int NW, bool STAGE_ALL = false, int E = gauss_elems<MP>(), int LIMIT = GAUSS_LDS_BYTES>
 struct GaussCfg {
   static constexpr int NCB = (V == GV_UGRADC) ? 2 : ((V == GV_PAIRS || V == GV_CURL_CROSS) ? 6 : 0);
   static constexpr bool ALL =
       STAGE_ALL && V != GV_PAIRS && GaussLds<MP, NW, 4, NCB, E>::TOTAL * 16 <= GAUSS_LDS_BYTES;
   // chunk buffers when not staging all at once: two where they fit
-  static constexpr int NBUF = GaussLds<MP, NW, 2, NCB, E>::TOTAL * 16 <= GAUSS_LDS_BYTES ? 2 : 1;
+  static constexpr int NBUF = GaussLds<MP, NW, 2, NCB, E>::TOTAL * 16 <= LIMIT ? 2 : 1;
   using LY = GaussLds<MP, NW, ALL ? 4 : NBUF, NCB, E>;
-  static_assert(LY::TOTAL * 16 <= GAUSS_LDS_BYTES, "LDS of the work-group");
+  static_assert(LY::TOTAL * 16 <= LIMIT, "LDS of the work-group");
 };
+
+// Layouts of the point tiles and of the element sums: two work-groups share a
+// CU where a wave holds one group in 4 waves.
+template <int MP, int V>
+using GaussHalfCfg = GaussCfg<MP, V, 4, false, 128 / MP, GAUSS_LDS_BYTES / 2>;
+template <int MP, int V>
+using GaussPtCfg = GaussCfg<MP, V, GAUSS_PT_WAVES, false, gauss_pt_elems<MP>(), GAUSS_LDS_BYTES / 2>;
+template <int MP, int V>
+using GaussRhsCfg = GaussCfg<MP, V, gauss_rhs_waves<MP, V>(), false, gauss_rhs_elems<MP>(),
+                             gauss_rhs_half<MP>() ? GAUSS_LDS_BYTES / 2 : GAUSS_LDS_BYTES>;
 
 struct GaussGeom {
   const double* w;       // shape values at this Gauss point (LDS table)
@@ -497,7 +534,9 @@ SFX_DEV void gauss_prologue(const GaussArgs& a, int tid, int64_t e0, double2* sm
 template <int MP, int V, int NW, bool STAGE_ALL = false, bool RHS = false, bool PT = false, int E = gauss_elems<MP>()>
 SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem) {
   using S = Shape<MP>;
-  using CFG = GaussCfg<MP, V, NW, STAGE_ALL, E>;
+  constexpr bool HALF = !PT && !RHS && E < gauss_elems<MP>();
+  using CFG = std::conditional_t<PT, GaussPtCfg<MP, V>, std::conditional_t<RHS, GaussRhsCfg<MP, V>,
+              std::conditional_t<HALF, GaussHalfCfg<MP, V>, GaussCfg<MP, V, NW, STAGE_ALL, E>>>>;
   using LY = typename CFG::LY;
   constexpr bool ALL = CFG::ALL;
   constexpr int L = S::L, PW = S::PW, NGR = point_groups<MP, E>(), NG = PT ? 1 : groups_per_wave<MP, E, NW>();
@@ -505,8 +544,8 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
   constexpr int NSIG = GVT<V>::NSIG, NO = GVT<V>::NOUT;
   // Outputs staged in LDS and stored in whole runs of the work-group's points
   // per plane (one group per wave): the point tiles, and the single-pass
-  // (curl a) x b of the pass lists (tangent at 50,000 triangles, M = 32:
-  // 4.22 -> 4.06 ms; neutral at M = 64; u.grad c gains nothing at M = 64).
+  // (curl a) x b (tangent 4 % faster at M = 32, neutral at 64; u.grad c gains
+  // nothing at 64).
   constexpr bool SOUT = !RHS && !STAGE_ALL && NG == 1 && (PT || V == GV_CURL_CROSS);
   constexpr int NF = 4 * NSIG;
   constexpr int NOC = (NO + 1) / 2;
@@ -544,16 +583,15 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
   }
 
   // The first chunks' loads depend on the connectivity alone: they leave with
-  // those of the tables, ahead of the first barrier and the geometry, and a
-  // chunk is two ahead of its use where a second work-group shares the CU or
-  // two fields are staged (forward term at 200,704 triangles, M = 64, 3.81 ->
-  // 3.61 ms, of whose 59,000 cycles a wave spent 19,000 waiting for chunks;
-  // tangent at 99,856 triangles, M = 32, 3.28 -> 3.23 ms, with one ahead 3.24).
-  // The element sums keep one ahead: two take 6.79 ms against 6.54 at 90,300
-  // triangles, M = 100, and 0.754 against 0.745 for u.grad c, M = 24.
+  // those of the tables, ahead of the first barrier and the geometry, and the
+  // cross-curl's point tiles and (curl a) x b keep two chunks in flight (forward
+  // term at 200,704 triangles, M = 64, 3.81 -> 3.61 ms, of whose 59,000 cycles a
+  // wave spent 19,000 waiting for chunks; tangent at 99,856 triangles, M = 32,
+  // 2.65 -> 2.59 ms).  The element sums keep one ahead: two take 5.60 ms against
+  // 5.50 at 90,300 triangles, M = 100.
   constexpr bool EARLY = !ALL && V != GV_PAIRS;
   constexpr int NCB = (V == GV_UGRADC) ? 2 : 6;
-  constexpr int DEP = ALL ? 4 : (PT || V == GV_CURL_CROSS) ? 2 : 1;   // chunks in registers
+  constexpr int DEP = ALL ? 4 : ((PT && V == GV_CROSS_CURL) || V == GV_CURL_CROSS) ? 2 : 1;   // chunks in registers
   NodalSlots<MP, NW, E> slots;
   NodalFetch<6, MP, NW, E> fa[DEP];
   NodalFetch<NCB, MP, NW, E> fb[DEP];
@@ -751,7 +789,7 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
         // the work-group's outputs go through LDS (st[P * SR + lp] for
         // output plane P = 2o + h + 2 NO m), so that the stores below write
         // whole runs of the tile's points per plane
-        constexpr int TP = PT ? NW * PW : 7 * E, SR = TP + 1;
+        constexpr int TP = PT ? NW * PW : NGR * PW, SR = TP + 1;
         static_assert(2 * NO * MP * SR <= LY::NODAL + NW * LY::RW, "output staging");
         double* st = big;
         const int lp = wave * PW + pt;
@@ -799,14 +837,14 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
   }
   if constexpr (SOUT) {
     // a thread keeps one point and takes every L-th plane
-    constexpr int TP = PT ? NW * PW : 7 * E, SR = TP + 1;
+    constexpr int TP = PT ? NW * PW : NGR * PW, SR = TP + 1;
     static_assert(NT == TP * L, "planes per round");
     const int lp = tid % TP, P0 = tid / TP;
     const int64_t pg = p0 + lp;
     const double* st = big + P0 * SR + lp;
     double* o = a.Vout + pg + a.G * (int64_t)P0;
     SFX_SYNC();
-    if (pg < 7 * a.me) {
+    if (pg < 7 * a.me && (PT || lp < 7 * E)) {
 #pragma unroll 4
       for (int P = P0; P < 2 * NO * a.M; P += L, st += L * SR, o += a.G * L) {
         SFX_CHECK("out stage read", st - big, 2 * NO * MP * SR);

@@ -128,14 +128,20 @@ extern "C" int emu_fftprod(int op, const double* V1, const double* V2, double* V
 
 template <int MP, int V>
 static void emu_gauss_mp(const GaussArgs& a) {
-  if constexpr (gauss_point_tiles<MP, V>()) {   // as the GPU launcher
-    constexpr int NW = GAUSS_PT_WAVES;
-    run_grid(gauss_blocks<MP, V, NW>(a.me), 64 * NW, GaussCfg<MP, V, NW>::LY::TOTAL,
-             [&](int t, int64_t b, double2* s) { gauss_body<MP, V, NW, false, false, true>(a, t, b, s); });
-  } else {
+  // as the GPU launcher
+  const bool whole = gauss_take_whole<MP, V>(a.me) || !(gauss_point_tiles<MP, V>() || gauss_half<MP, V>());
+  const int64_t nblk = whole ? gauss_whole_blocks<MP>(a.me) : gauss_blocks<MP, V>(a.me);
+  if (whole) {
     constexpr int NW = gauss_waves<MP, V>();
-    run_grid(gauss_blocks<MP, V, NW>(a.me), 64 * NW, GaussCfg<MP, V, NW>::LY::TOTAL,
+    run_grid(nblk, 64 * NW, GaussCfg<MP, V, NW>::LY::TOTAL,
              [&](int t, int64_t b, double2* s) { gauss_body<MP, V, NW>(a, t, b, s); });
+  } else if constexpr (gauss_point_tiles<MP, V>()) {
+    run_grid(nblk, 64 * GAUSS_PT_WAVES, GaussPtCfg<MP, V>::LY::TOTAL, [&](int t, int64_t b, double2* s) {
+      gauss_body<MP, V, GAUSS_PT_WAVES, false, false, true, gauss_pt_elems<MP>()>(a, t, b, s);
+    });
+  } else if constexpr (gauss_half<MP, V>()) {
+    run_grid(nblk, 256, GaussHalfCfg<MP, V>::LY::TOTAL,
+             [&](int t, int64_t b, double2* s) { gauss_body<MP, V, 4, false, false, false, 128 / MP>(a, t, b, s); });
   }
 }
 
@@ -896,7 +902,7 @@ static void emu_nl_rhs_mp(const GaussArgs& a) {
   constexpr int NW = gauss_rhs_waves<MP, GV_CROSS_CURL>();
   constexpr int E = gauss_rhs_elems<MP>();
   const int64_t nblk = (a.me + E - 1) / E;
-  run_grid(nblk, 64 * NW, GaussCfg<MP, GV_CROSS_CURL, NW, false, E>::LY::TOTAL,
+  run_grid(nblk, 64 * NW, GaussRhsCfg<MP, GV_CROSS_CURL>::LY::TOTAL,
            [&](int t, int64_t b, double2* s) { gauss_body<MP, GV_CROSS_CURL, NW, false, true, false, E>(a, t, b, s); });
 }
 
@@ -952,7 +958,7 @@ static void emu_nl_qs00_mp(const GaussArgs& a) {
   constexpr int NW = gauss_rhs_waves<MP, GV_UGRADC>();
   constexpr int E = gauss_rhs_elems<MP>();
   const int64_t nblk = (a.me + E - 1) / E;
-  run_grid(nblk, 64 * NW, GaussCfg<MP, GV_UGRADC, NW, false, E>::LY::TOTAL,
+  run_grid(nblk, 64 * NW, GaussRhsCfg<MP, GV_UGRADC>::LY::TOTAL,
            [&](int t, int64_t b, double2* s) { gauss_body<MP, GV_UGRADC, NW, false, true, false, E>(a, t, b, s); });
 }
 
