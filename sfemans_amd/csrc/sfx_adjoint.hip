@@ -4,9 +4,9 @@
 namespace sfx {
 
 template <int MP, bool SPLIT>
-constexpr int adjoint_occupancy() { return adjoint_half<MP, SPLIT>() ? 2 : 1; }
+constexpr int adjoint_occupancy() { return AdjLds<MP, SPLIT, adjoint_waves<MP, SPLIT>()>::PARK ? 2 : 1; }
 
-template <int MP, bool SPLIT, int NW = ADJOINT_WAVES>
+template <int MP, bool SPLIT, int NW = adjoint_waves<MP, SPLIT>()>
 __global__ void __launch_bounds__(64 * NW)
 __attribute__((amdgpu_waves_per_eu(adjoint_occupancy<MP, SPLIT>(), adjoint_occupancy<MP, SPLIT>())))
 adjoint_kernel(AdjArgs a) {
@@ -21,7 +21,7 @@ __global__ void __launch_bounds__(GATHER_THREADS) adjoint_gather_kernel(GatherAr
 
 template <int MP, bool SPLIT>
 static hipError_t launch_mp(const AdjArgs& a, hipStream_t st) {
-  constexpr int NW = ADJOINT_WAVES;
+  constexpr int NW = adjoint_waves<MP, SPLIT>();
   constexpr int E = adjoint_elems<MP, SPLIT>();
   const int64_t nblk = (a.g.me + E - 1) / E;
   if (nblk == 0) return hipSuccess;

@@ -43,24 +43,29 @@ template <bool SPLIT> struct AdjRed { static constexpr int K = SPLIT ? 24 : 18; 
 // layout fits in half the LDS; elsewhere 4 waves with two groups each in 512
 // registers.  Half tiles against what stood there, convective form: 0.80 / 0.98
 // ms at MP = 4, 0.84 / 1.10 at 8 (both against 512 registers), 0.91 / 0.96 at 16,
-// 0.68 / 0.76 at 64, 0.86 / 0.94 at 128 (against 7 waves with one group each; a
+// 0.68 / 0.76 at 64 and 8.16 / 9.20 at 64 and 200,704 triangles (against 7 waves
+// with one group each, which stay at MP = 128: half tiles of one element read 56-byte
+// pieces of ybar and take 25.4 ms there against 22.6 at 200,704 triangles; a
 // wave waited 13,000 of 100,000 cycles at the barrier before the sums, three SIMDs
 // holding two waves and one holding one); split form, against 512 registers: 1.18
 // / 1.79 ms at MP = 8, 1.27 / 1.64 at 16, 1.31 / 1.68 at 32, 1.33 / 1.79 at 64.
 template <int MP, bool SPLIT>
-constexpr bool adjoint_half() { return SPLIT ? MP >= 8 && MP <= 64 : MP <= 128; }
+constexpr bool adjoint_half() { return MP <= 64 && (!SPLIT || MP >= 8); }
 template <int MP, bool SPLIT>
 constexpr int adjoint_elems() { return adjoint_half<MP, SPLIT>() ? 128 / MP : gauss_elems<MP>(); }
-constexpr int ADJOINT_WAVES = 4;
+// Whole tiles: the convective form at MP = 128 in the parking form on 7 waves.
+template <int MP, bool SPLIT>
+constexpr int adjoint_waves() { return !SPLIT && MP == 128 ? 7 : 4; }
 
 template <int MP, bool SPLIT, int NW>
 struct AdjLds {
   using LY = GaussLds<MP, NW, 1, 6, adjoint_elems<MP, SPLIT>()>;
   static constexpr int NT = 64 * NW;
-  // Parking (half tiles, 256 registers per lane): base spectra wait in LDS
+  // Parking (256 registers per lane): base spectra wait in LDS
   // while pbar is formed, and pbar waits in LDS during the base-field
   // transforms, so that neither is spilled to scratch.
-  static constexpr bool PARK = adjoint_half<MP, SPLIT>();
+  static constexpr bool HALF = adjoint_half<MP, SPLIT>();
+  static constexpr bool PARK = HALF || NW > 4;
   // signals transformed together; the per-wave region also holds the partner
   // swap of the base fields (64 x 12 doubles) and, in the 512-register form,
   // of ybar (64 x 24)
@@ -87,7 +92,7 @@ struct AdjLds {
   // parked doubles per lane: PK1 in the staging area (idle once the base
   // fields are interpolated; slot f of lane t at f * NT + t), PK2 past BIGD
   // in what is left of the work-group's share of the 160 KB
-  static constexpr int LDS_DOUBLES = (PARK ? 80 : 160) * 1024 / 8;
+  static constexpr int LDS_DOUBLES = (HALF ? 80 : 160) * 1024 / 8;
   static constexpr int PK1 = PARK ? NODAL / NT : 0;
   static constexpr int PK2 = PARK ? (LDS_DOUBLES - 2 * LY::BIG - BIGD) / NT : 0;
   static constexpr int PK = PK1 + PK2;

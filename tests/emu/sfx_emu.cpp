@@ -337,7 +337,7 @@ extern "C" int emu_rhs_ns(const int32_t* jj, const double* rr, int64_t me, int64
 
 template <int MP, bool SPLIT>
 static void emu_adjoint_mp(const AdjArgs& A) {
-  constexpr int NW = ADJOINT_WAVES;
+  constexpr int NW = adjoint_waves<MP, SPLIT>();
   constexpr int E = adjoint_elems<MP, SPLIT>();
   const int64_t nblk = (A.g.me + E - 1) / E;
   run_grid(nblk, 64 * NW, AdjLds<MP, SPLIT, NW>::TOTAL,
