@@ -1,6 +1,6 @@
 """Results of the host-pointer entry points, copied back in page-locked chunks
 of 1 MB (ring of 4): the same bytes as the device-pointer entry points write,
-for results of less than two chunks (one hipMemcpy), of whole and of ragged
+for results of less than two chunks or more than 32 (one hipMemcpy), of whole and of ragged
 chunk counts, of more chunks than the ring has, and after the ring was given
 back.
 """
@@ -22,7 +22,7 @@ def gpu():
 
 
 # M = 2: 96 bytes of result per point, 2 MB at 21845.33 points
-@pytest.mark.parametrize("npt", [21845, 21846, 32768, 43690, 43691, 54613, 54614, 98304, 120001])
+@pytest.mark.parametrize("npt", [21845, 21846, 32768, 43690, 43691, 54613, 54614, 98304, 120001, 349525, 349526])
 @pytest.mark.parametrize("pinned", [False, True])
 def test_host_result_is_the_device_result(npt, pinned):
     M = 2
