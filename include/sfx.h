@@ -119,7 +119,12 @@ int sfx_fft_tensor_dcl_dev(const double* V1_in, const double* V2_in, double* V_o
  * scratch (up to 2 * outputs * m_max_pad * np doubles) per (device, stream):
  * calls on different streams may overlap.  A call that must grow it waits
  * for its stream first, so under HIP graph capture make one call of the
- * largest size beforehand.  sfx_stream_release frees a stream's scratch.
+ * largest size (2 * outputs * m_max_pad * np) beforehand on that stream, and
+ * one with each (m_max_c, m_max_pad), whose tables are built at their first
+ * use.  Calls that run without the scratch (on the matrix cores) reserve it
+ * all the same, on any stream but the null stream and where the memory is
+ * there, so any of these products serves as that call.
+ * sfx_stream_release frees a stream's scratch.
  * The host-pointer forms stage their arrays in per-device buffers: call
  * them from one host thread at a time per device.
  * ------------------------------------------------------------------------- */

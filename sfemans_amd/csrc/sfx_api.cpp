@@ -129,6 +129,38 @@ int stream_scratch(int slot, size_t bytes, hipStream_t st, void** out) {
   return SFX_OK;
 }
 
+// Room in a slot for later calls, asked for by a call that runs without it: a
+// slot then holds what the largest call so far could need, whichever kernels
+// it took, so that calls captured after it allocate nothing.  No error: where
+// the memory cannot be had the slot stays as it is, and only a call that uses
+// it is refused.  Nothing is done for a stream under capture, nor for the null
+// stream, which cannot be captured; other streams' captures are not disturbed
+// (relaxed mode).
+void stream_scratch_reserve(int slot, size_t bytes, hipStream_t st) {
+  int dev = 0;
+  if (!st || slot < 0 || slot >= N_STAGING || hipGetDevice(&dev) != hipSuccess) return;
+  std::lock_guard<std::mutex> lk(g_mu);
+  Staging& s = g_stream_scratch[std::make_pair(dev, (uintptr_t)st)];
+  if (s.n[slot] >= bytes) return;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  hipError_t e = hipStreamIsCapturing(st, &cap);
+  if (e == hipSuccess && cap == hipStreamCaptureStatusNone &&
+      (e = hipThreadExchangeStreamCaptureMode(&mode)) == hipSuccess) {
+    void* p = nullptr;
+    e = hipMalloc(&p, bytes);
+    if (e == hipSuccess && s.p[slot] && (e = hipStreamSynchronize(st)) == hipSuccess) (void)hipFree(s.p[slot]);
+    if (e == hipSuccess) {
+      s.p[slot] = p;
+      s.n[slot] = bytes;
+    } else if (p) {
+      (void)hipFree(p);
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  if (e != hipSuccess) (void)hipGetLastError();   // not left for the launch's check
+}
+
 int release_stream_scratch(hipStream_t st) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);

@@ -35,6 +35,7 @@ void clear_err();
 int get_twiddles(int MP, Twiddles* tw);
 int staging(int slot, size_t bytes, void** out);
 int stream_scratch(int slot, size_t bytes, hipStream_t st, void** out);
+void stream_scratch_reserve(int slot, size_t bytes, hipStream_t st);
 int release_stream_scratch(hipStream_t st);
 hipError_t copy_out(void* h, const void* d, size_t n);
 hipError_t release_hostcopy();

@@ -70,14 +70,20 @@ static int exact_prepare(const char* nm, ExactArgs& a, int op, int64_t np, int M
   if (rc) return rc;
   // EX_EVISC's products are those of EX_GRADMOM on its last nine inputs
   if (!exact_mm_use(op == EX_EVISC ? EX_GRADMOM : op, a)) a.mmtab = nullptr;
-  if (a.mmtab) return SFX_OK;   // no scratch
+  const int64_t n_W = 2 * (int64_t)a.nout * (a.K + 1) * np;
+  if (a.mmtab) {
+    // no scratch, but a later call that is no larger may take the two-pass
+    // kernels (outputs over inputs, exact_mm_use) and be under capture
+    stream_scratch_reserve(SLOT_EX_W, (size_t)n_W * 8, st);
+    return SFX_OK;
+  }
   void* w = nullptr;
   if (exact_is_reduction(op)) {
     const int64_t nb = exact_grid_blocks(op, a.nin, np, a.K);
     if ((rc = stream_scratch(SLOT_EX_W, (size_t)(nb > 0 ? nb : 1) * 8, st, &w))) return rc;
     a.pmax = (double*)w;
   } else {
-    a.n_W = 2 * (int64_t)a.nout * (a.K + 1) * np;
+    a.n_W = n_W;
     if ((rc = stream_scratch(SLOT_EX_W, (size_t)(a.n_W > 0 ? a.n_W : 1) * 8, st, &w))) return rc;
     a.W = (double*)w;
   }
