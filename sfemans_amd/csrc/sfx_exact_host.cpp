@@ -68,8 +68,7 @@ static int exact_prepare(const char* nm, ExactArgs& a, int op, int64_t np, int M
   exact_setup_sizes(a, np, M, m_max_pad);
   int rc = exact_tables(M, a.K, &a.ctab, &a.rtab, &a.mmtab);
   if (rc) return rc;
-  // EX_EVISC's products are those of EX_GRADMOM on its last nine inputs
-  if (!exact_mm_use(op == EX_EVISC ? EX_GRADMOM : op, a)) a.mmtab = nullptr;
+  if (!exact_mm_use(op, a)) a.mmtab = nullptr;
   const int64_t n_W = 2 * (int64_t)a.nout * (a.K + 1) * np;
   if (a.mmtab) {
     // no scratch, but a later call that is no larger may take the two-pass

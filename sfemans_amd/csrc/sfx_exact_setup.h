@@ -79,24 +79,100 @@ inline bool exact_mm_disjoint(const ExactArgs& a) {
   return true;
 }
 
-// Whether a product runs on the matrix-core kernel.  Times, two-pass kernels /
-// matrix-core kernel in us, on 60,000 points unless said otherwise:
-// - its exact form (M <= 64 on a grid of 3/2 as many angle pairs) is faster at
-//   every number of points: v / s 154 / 76 at M = 32, 464 / 236 at M = 64 and
-//   59 / 19 on 500 points, tension tensor 1101 / 767 at M = 64;
-// - but blocks of 16 modes are mostly empty for a few modes: v / s 19 / 20 and
-//   tension 37 / 75 at M = 4, tension 65 / 78 and v / s 30 / 22 at M = 8;
-// - the general form repeats the synthesis for the second half of the modes:
-//   v / s 662 / 707 at M = 80 and 1148 / 1305 at M = 112, but on 500 points,
-//   where the two-pass kernels leave the chip idle, 81 / 30 and 146 / 49;
-// - the analysis alone (EX_FROMREAL) has no synthesis: 238 / 87 at M = 80.
+// Products that stay on the two-pass kernels though the matrix-core kernel has
+// their sizes: with M modes in whole blocks of 16 and m_max_pad angles in
+// blocks of 16, the share of useful products, f = M m_max_pad / (256 blocks),
+// is small for a few modes and for a mode count a little above a multiple of
+// 16, and the operation runs on every padded angle (and, for the tension and
+// the entropy viscosities, again for each output).  Below some number of
+// points the two-pass kernels are two launches that leave the chip idle, and
+// the matrix-core kernel is faster all the same; with a scratch array larger
+// than the last-level cache (256 MB, which S, D and the inputs share) they
+// fall behind again.  A product takes the two-pass kernels if one of its
+// lines holds: more than points + slope f points, f below the line's, at most
+// `scratch` MB of S and D, at least `modes` modes.  Times, two-pass /
+// matrix-core kernel in us, on both sides of the lines:
+//   tension   M = 2: 12 / 12 on 8,190 points, 55 / 289 on 262,136; M = 8: 33 / 23 on 16,380, 55 / 59 on 49,140;
+//             M = 12: 43 / 38 on 16,380, 58 / 69 on 32,767, 297 / 266 on 131,068; M = 14: 348 / 280 on 131,068
+//   compressive entropy viscosity   M = 2: 14 / 11 on 8,190, 14 / 46 on 65,534; M = 10: 130 / 110 on 131,068;
+//             M = 12: 34 / 28 on 16,380, 168 / 203 on 131,068; M = 24: 91 / 108 on 32,767, 442 / 450 on 131,068
+//   entropy viscosity   M = 6: 38 / 25 on 8,190, 82 / 99 on 65,534, 372 / 421 on 262,136; M = 8: 115 / 102 on 65,534
+//   level-set compression   M = 17: 39 / 28 on 12,285, 136 / 174 on 131,068; M = 38: 183 / 159 on 49,140
+//   Heaviside of 2 interfaces   M = 12: 45 / 38 on 131,068; M = 24: 45 / 28 on 32,767, 77 / 91 on 131,068;
+//             of 4   M = 10: 30 / 21 on 49,140, 58 / 68 on 196,602
+//   the others, only for a few modes   v / s M = 2: 12 / 10 on 32,767, 24 / 69 on 262,136, M = 6: 73 / 70 there;
+//             gradients M = 4: 18 / 14 on 16,380, 38 / 44 on 65,534; division M = 2: 11 / 10 on 65,534, 12 / 28 on
+//             262,136
+struct ExactMmLine {
+  int op, nin;                       // nin: 0 for any
+  int modes;
+  double points, slope, f, scratch;  // points and slope in units of 1024
+};
+constexpr double EXACT_MM_ANY = 1e30;
+constexpr ExactMmLine EXACT_MM_LINES[] = {
+    {EX_TENSION, 0, 1, 8, 64, 0.28, EXACT_MM_ANY},
+    {EX_TENSION, 0, 1, 24, 0, 0.50, 145},
+    {EX_TENSION, 0, 17, 20, 0, 0.57, 125},
+    {EX_COMPR, 0, 1, 16, 0, 0.40, EXACT_MM_ANY},
+    {EX_COMPR, 0, 12, 16, 0, 0.52, EXACT_MM_ANY},
+    {EX_COMPR, 0, 12, 24, 0, 0.58, 80},
+    {EX_COMPR, 0, 17, 22, 0, 0.61, 80},
+    {EX_EVISC, 0, 1, 8, 128, 0.22, EXACT_MM_ANY},
+    {EX_EVISC, 0, 1, 8, 128, 0.65, 100},
+    {EX_CLS, 0, 1, 34, 120, 0.40, EXACT_MM_ANY},
+    {EX_CLS, 0, 9, 56, 0, 0.58, EXACT_MM_ANY},
+    {EX_CLS, 0, 17, 40, 0, 0.69, EXACT_MM_ANY},
+    {EX_HEAVI, 1, 1, 96, 0, 0.10, EXACT_MM_ANY},
+    {EX_HEAVI, 2, 1, 96, 0, 0.22, EXACT_MM_ANY},
+    {EX_HEAVI, 2, 17, 63, 0, 0.65, EXACT_MM_ANY},
+    {EX_HEAVI, 3, 1, 48, 0, 0.12, EXACT_MM_ANY},
+    {EX_HEAVI, 3, 1, 100, 0, 0.25, EXACT_MM_ANY},
+    {EX_HEAVI, 3, 1, 160, 0, 0.50, EXACT_MM_ANY},
+    {EX_HEAVI, 3, 12, 48, 0, 0.65, EXACT_MM_ANY},
+    {EX_HEAVI, 3, 17, 31, 0, 0.80, EXACT_MM_ANY},
+    {EX_HEAVI, 4, 1, 40, 0, 0.12, EXACT_MM_ANY},
+    {EX_HEAVI, 4, 1, 66, 0, 0.60, EXACT_MM_ANY},
+    {EX_HEAVI, 4, 12, 48, 0, 0.65, EXACT_MM_ANY},
+    {EX_HEAVI, 4, 17, 31, 0, 0.78, EXACT_MM_ANY},
+    {EX_GRADMOM, 0, 1, 16, 96, 0.10, EXACT_MM_ANY},
+    {EX_ENTRO, 0, 1, 32, 256, 0.14, EXACT_MM_ANY},
+    {EX_ETA3, 0, 1, 48, 256, 0.10, EXACT_MM_ANY},
+    {EX_SV2, 0, 1, 40, 128, 0.14, EXACT_MM_ANY},
+    {EX_SVCLAMP, 0, 1, 40, 128, 0.14, EXACT_MM_ANY},
+    {EX_DIV, 0, 1, 64, 512, 0.22, EXACT_MM_ANY},
+    {EX_DIV, 0, 17, 96, 0, 0.54, 80},
+    {EX_ETA, 0, 1, 96, 0, 0.05, EXACT_MM_ANY},
+    {EX_SQRT, 0, 1, 96, 0, 0.05, EXACT_MM_ANY},
+    {EX_CLAMP01, 0, 1, 96, 0, 0.05, EXACT_MM_ANY},
+    {EX_FROMREAL, 0, 1, 300, 0, 0.03, EXACT_MM_ANY}};
+
+inline bool exact_mm_two_pass(int op, const ExactArgs& a) {
+  const double f = a.M * (double)(a.K + 1) / (256.0 * exact_mm_mbn(a.M) * exact_mm_jbn(a.K));
+  const double mb = 16.0 * a.nout * (a.K + 1) * (double)a.np / (1 << 20);
+  for (const ExactMmLine& l : EXACT_MM_LINES)
+    if (l.op == op && (l.nin == 0 || l.nin == a.nin) && a.M >= l.modes && f < l.f && mb <= l.scratch &&
+        (double)a.np > 1024.0 * (l.points + l.slope * f))
+      return true;
+  return false;
+}
+
+// Whether a product runs on the matrix-core kernel (EX_EVISC: its two parts).
+// Its exact form (M <= 64 on a grid of 3/2 as many angle pairs) beside the
+// lines above.  The general form (more modes, other grids) repeats the
+// synthesis for the second half of the modes and is taken up to the number of
+// points where every product still gains (M = 80, v / s 76 / 30 us, tension
+// 130 / 86 on 2,044 points, but tension 137 / 164 on 4,088; v / s gains up to
+// some 32,000).  The analysis alone (EX_FROMREAL) has no synthesis: 238 / 87 on
+// 60,000 points at M = 80.
 inline bool exact_mm_use(int op, const ExactArgs& a) {
-  if (!exact_mm_has(op) || a.np <= 0 || !exact_mm_sizes(a.M, a.K) || !exact_mm_disjoint(a)) return false;
-  if (op == EX_FROMREAL) return true;
+  // EX_EVISC's products are those of EX_GRADMOM on its last nine inputs
+  if (!exact_mm_has(op == EX_EVISC ? EX_GRADMOM : op) || a.np <= 0 || !exact_mm_sizes(a.M, a.K) ||
+      !exact_mm_disjoint(a))
+    return false;
+  if (op == EX_FROMREAL) return !exact_mm_two_pass(op, a);
   const int jb = exact_mm_jb(exact_mm_mb(a.M)), jbn = exact_mm_jbn(a.K);
   if (a.M > 64 || (jbn != jb && jbn != jb - 1)) return a.np <= 2048;
-  const bool few = a.M <= 4 || (a.M <= 8 && (op == EX_TENSION || op == EX_COMPR));
-  return !few || a.np <= 16384;
+  return !exact_mm_two_pass(op, a);
 }
 
 inline void exact_setup_sizes(ExactArgs& a, int64_t np, int M, int m_max_pad) {

@@ -172,8 +172,8 @@ namespace sfx {
 hipError_t launch_fftprod(int, const FftProdArgs&, hipStream_t) { return hipSuccess; }
 hipError_t launch_exact(int op, const ExactArgs& a, double*, hipStream_t) {
   ++g_count[a.mmtab ? "matrix" : "twopass"];
-  // the two-pass kernels fill their whole scratch
-  if (!a.mmtab && !exact_is_reduction(op)) memset(a.W, 0, (size_t)a.n_W * sizeof(double));
+
+
   return hipSuccess;
 }
 hipError_t launch_exact_emom(const ExactArgs&, double*, hipStream_t) { return hipSuccess; }

@@ -27,9 +27,9 @@ def routes(L):
 
 
 # (warm-up, captured) as (np, M, in place): a call of the same size whose output is its input; more than
-# 2,048 points of more than 64 modes; more than 16,384 points of few modes (smaller in scratch than the warm-up)
+# 2,048 points of more than 64 modes; few modes on many points (smaller in scratch than the warm-up)
 CASES = [((3000, 16, False), (3000, 16, True)), ((3000, 16, False), (2999, 16, True)),
-         ((2048, 80, False), (2049, 79, False)), ((16384, 8, False), (16385, 4, False))]
+         ((2048, 80, False), (2049, 79, False)), ((70000, 8, False), (60000, 4, False))]
 
 
 @pytest.mark.parametrize("warm,cap", CASES)
