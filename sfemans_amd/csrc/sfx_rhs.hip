@@ -11,10 +11,10 @@ __global__ void __launch_bounds__(256) rhs_elem_kernel(RhsArgs a) {
   rhs_elem_body(a, xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x);
 }
 
-template <bool TENSOR>
+template <bool TENSOR, int MC>
 __global__ void __launch_bounds__(RNS_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) rhs_ns_tile_kernel(RhsArgs a) {
   __shared__ __attribute__((aligned(16))) double smem[rns_smem_doubles<TENSOR>()];
-  rhs_ns_tile_body<TENSOR>(a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x), smem);
+  rhs_ns_tile_body<TENSOR, MC>(a, threadIdx.x, xcd_block(blockIdx.x, gridDim.x), smem);
 }
 
 // The Gauss values of the NS right-hand side before the penalty product.
@@ -63,13 +63,20 @@ hipError_t launch_qs00_gather(const RhsArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <int MC>
+static void rns_launch(const RhsArgs& a, int64_t nt, hipStream_t st) {
+  if (a.tens) hipLaunchKernelGGL((rhs_ns_tile_kernel<true, MC>), dim3((unsigned)nt), dim3(RNS_THREADS), 0, st, a);
+  else hipLaunchKernelGGL((rhs_ns_tile_kernel<false, MC>), dim3((unsigned)nt), dim3(RNS_THREADS), 0, st, a);
+}
+
 // Full NS right-hand side fused with its element share, then the gather.
 hipError_t launch_rhs_ns(const RhsArgs& a, hipStream_t st) {
-  const int64_t nn = a.np * a.M, nt = a.me > 0 && a.M > 0 ? rns_blocks(a.me, a.M) : 0;
+  const int mc = rns_modes(a.me, a.M);
+  const int64_t nn = a.np * a.M, nt = a.me > 0 && a.M > 0 ? rns_blocks(a.me, a.M, mc) : 0;
   if (nt > 0x7fffffffLL) return hipErrorInvalidValue;
   if (nt > 0) {
-    if (a.tens) hipLaunchKernelGGL(rhs_ns_tile_kernel<true>, dim3((unsigned)nt), dim3(RNS_THREADS), 0, st, a);
-    else hipLaunchKernelGGL(rhs_ns_tile_kernel<false>, dim3((unsigned)nt), dim3(RNS_THREADS), 0, st, a);
+    if (mc == RNS_FEW) rns_launch<RNS_FEW>(a, nt, st);
+    else rns_launch<RNS_MC>(a, nt, st);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nn == 0) return e;

@@ -134,14 +134,14 @@ SFX_DEV void rhs_elem_body(const RhsArgs& a, int64_t gid) {
 // The Gauss array rhs_gauss is never stored.
 //
 // What bounds it: HBM (rotv_v and the tensor are 192 bytes per Gauss point and
-// mode).  A work-group takes RNS_E elements and RNS_MC modes of them, one mode
+// mode).  A work-group takes RNS_E elements and MC modes of them, one mode
 // at a time: one thread per Gauss point loads rotv_v and the tensor (224
 // consecutive points of each plane, whole lines), one per (element, node) the
 // nodal fields, which are added at the nodes (V1m + ff, P + P_inc) and
 // interpolated from LDS; each point's weights of the shape values and of the
 // reference derivatives (18 numbers, as in the adjoint) go to LDS, and one
-// thread per (element, component) sums them for the six nodes, keeping RNS_MC
-// modes so that it stores 64-byte runs.  (One thread per (element, mode) with all
+// thread per (element, component) sums them for the six nodes, keeping MC
+// modes so that it stores 64-byte runs (MC = RNS_MC).  (One thread per (element, mode) with all
 // of its fields in registers took 418 registers, one wave per SIMD, and each of
 // its loads touched 40 lines: 1.4 TB/s, 6.15 ms with the gather at 102,720
 // triangles, M = 48, against 3.04 ms, 3.8 TB/s in this kernel.)
@@ -151,15 +151,24 @@ constexpr int RNS_EROW = 6 * 8 + 2;            // doubles per element of the sta
 constexpr int RNS_SK = RNS_PT + 2;             // doubles per weight
 template <bool TENSOR>
 constexpr int rns_smem_doubles() { return 2 * RNS_E * RNS_EROW + (TENSOR ? 18 : 6) * RNS_SK + 128; }
-inline int64_t rns_blocks(int64_t me, int M) {
-  return ((me + RNS_E - 1) / RNS_E) * (int64_t)((M + RNS_MC - 1) / RNS_MC);
+inline int64_t rns_blocks(int64_t me, int M, int MC) {
+  return ((me + RNS_E - 1) / RNS_E) * (int64_t)((M + MC - 1) / MC);
 }
+// Modes per work-group: RNS_MC, or 2 where that would leave CUs idle while the
+// others work through eight modes in series (two work-groups share a CU).  With
+// the gather, without the tensor, one thread per (element, mode) / 8 modes / 2
+// modes: 26.5 / 28.5 / 14.9 us at 400 triangles, M = 8 (13 work-groups of 8), 107
+// / 114 / 104 at M = 128 (208), 62.8 / 57.9 / 52.0 at 3,192, M = 24 (300), but 65.6
+// / 65.8 at M = 32 (400) with 8 / 2 modes; with the tensor 67.8 / 61.5 (300) and 76.1
+// / 78.7 (400).
+constexpr int RNS_FEW = 2, RNS_FULL = 384;
+inline int rns_modes(int64_t me, int M) { return rns_blocks(me, M, RNS_MC) < RNS_FULL ? RNS_FEW : RNS_MC; }
 
-template <bool TENSOR>
+template <bool TENSOR, int MC>
 SFX_DEV void rhs_ns_tile_body(const RhsArgs& a, int tid, int64_t bid, double* smem) {
-  const int nmc = (a.M + RNS_MC - 1) / RNS_MC;
+  const int nmc = (a.M + MC - 1) / MC;
   const int64_t e0 = (bid / nmc) * RNS_E;      // the mode chunks of one set of elements are neighbours
-  const int m0 = (int)(bid % nmc) * RNS_MC, m1 = m0 + RNS_MC < a.M ? m0 + RNS_MC : a.M;
+  const int m0 = (int)(bid % nmc) * MC, m1 = m0 + MC < a.M ? m0 + MC : a.M;
   double* nod = smem;                          // two buffers: a slow thread still reads the other mode's
   double* red = nod + 2 * RNS_E * RNS_EROW;
   double* tab = red + (TENSOR ? 18 : 6) * RNS_SK;
@@ -191,14 +200,14 @@ SFX_DEV void rhs_ns_tile_body(const RhsArgs& a, int tid, int64_t bid, double* sm
     iray = 1.0 / ray;
     wl = a.wgt[p];
   }
-  double acc[RNS_MC][6];
+  double acc[MC][6];
 #pragma unroll
-  for (int q = 0; q < RNS_MC; ++q)
+  for (int q = 0; q < MC; ++q)
 #pragma unroll
     for (int i = 0; i < 6; ++i) acc[q][i] = 0.0;
 
 #pragma unroll
-  for (int q = 0; q < RNS_MC; ++q) {
+  for (int q = 0; q < MC; ++q) {
     const int m = m0 + q;
     if (m >= m1) continue;                     // uniform over the work-group
     // ---- loads of this mode
@@ -340,7 +349,7 @@ SFX_DEV void rhs_ns_tile_body(const RhsArgs& a, int tid, int64_t bid, double* sm
     for (int n = 0; n < 6; ++n) {
       const int64_t o = ((6 * (e0 + ke) + n) * 6 + kc) * (int64_t)a.M + m0;
 #pragma unroll
-      for (int q = 0; q < RNS_MC; ++q) {
+      for (int q = 0; q < MC; ++q) {
         if (m0 + q >= m1) continue;
         SFX_CHECK("elo store", o + q, a.n_elo);
         a.elo[o + q] = acc[q][n];

@@ -300,6 +300,20 @@ extern "C" int emu_rhs_ns_gauss(const int32_t* jj, const double* rr, int64_t me,
   return 0;
 }
 
+template <int MC>
+static void emu_rns_elems(const RhsArgs& a) {
+  if (a.tens)
+    run_grid(rns_blocks(a.me, a.M, MC), RNS_THREADS, (rns_smem_doubles<true>() + 1) / 2, [&](int t, int64_t b, double2* sm) {
+      rhs_ns_tile_body<true, MC>(a, t, b, reinterpret_cast<double*>(sm));
+    });
+  else
+    run_grid(rns_blocks(a.me, a.M, MC), RNS_THREADS, (rns_smem_doubles<false>() + 1) / 2, [&](int t, int64_t b, double2* sm) {
+      rhs_ns_tile_body<false, MC>(a, t, b, reinterpret_cast<double*>(sm));
+    });
+}
+
+extern "C" int emu_rns_modes(int64_t me, int M) { return rns_modes(me, M); }
+
 extern "C" int emu_rhs_ns(const int32_t* jj, const double* rr, int64_t me, int64_t np, const int32_t* lm, int M,
                           const double* rotv, const double* V1m, const double* ff, const double* P,
                           const double* Pinc, const double* tens, double* v145, double* v236) {
@@ -321,12 +335,12 @@ extern "C" int emu_rhs_ns(const int32_t* jj, const double* rr, int64_t me, int64
   a.n_rhs = a.G * 6 * (int64_t)M; a.n_v1m = a.n_fsrc = np * 6 * (int64_t)M; a.n_pres = a.n_pinc = np * 2 * (int64_t)M;
   a.n_tens = 3 * a.n_rhs;
   a.n_out = np * 3 * (int64_t)M; a.n_elo = 36 * me * (int64_t)M;
-  if (tens)
-    run_grid(rns_blocks(me, M), RNS_THREADS, (rns_smem_doubles<true>() + 1) / 2,
-             [&](int t, int64_t b, double2* sm) { rhs_ns_tile_body<true>(a, t, b, reinterpret_cast<double*>(sm)); });
-  else
-    run_grid(rns_blocks(me, M), RNS_THREADS, (rns_smem_doubles<false>() + 1) / 2,
-             [&](int t, int64_t b, double2* sm) { rhs_ns_tile_body<false>(a, t, b, reinterpret_cast<double*>(sm)); });
+  // both forms, whichever the rule takes; their element sums are the same bits
+  emu_rns_elems<RNS_FEW>(a);
+  const std::vector<double> few = elo;
+  std::fill(elo.begin(), elo.end(), NAN);
+  emu_rns_elems<RNS_MC>(a);
+  if (std::memcmp(few.data(), elo.data(), sizeof(double) * 36 * me * M) != 0) return 1;
   run_grid((np + GATHER_NODES - 1) / GATHER_NODES, GATHER_THREADS, (gather_tile_doubles<6>() + 1) / 2,
            [&](int t, int64_t b, double2* sm) { rhs_gather_block(a, b, t, reinterpret_cast<double*>(sm)); });
   return 0;
