@@ -150,7 +150,7 @@ constexpr int RNS_PT = 7 * RNS_E;              // Gauss points
 constexpr int RNS_EROW = 6 * 8 + 2;            // doubles per element of the staged nodal sums (8 per node)
 constexpr int RNS_SK = RNS_PT + 2;             // doubles per weight
 template <bool TENSOR>
-constexpr int rns_smem_doubles() { return 2 * RNS_E * RNS_EROW + (TENSOR ? 18 : 6) * RNS_SK + 128; }
+constexpr int rns_smem_doubles() { return RNS_E * RNS_EROW + (TENSOR ? 18 : 6) * RNS_SK + 128; }
 inline int64_t rns_blocks(int64_t me, int M, int MC) {
   return ((me + RNS_E - 1) / RNS_E) * (int64_t)((M + MC - 1) / MC);
 }
@@ -169,8 +169,10 @@ SFX_DEV void rhs_ns_tile_body(const RhsArgs& a, int tid, int64_t bid, double* sm
   const int nmc = (a.M + MC - 1) / MC;
   const int64_t e0 = (bid / nmc) * RNS_E;      // the mode chunks of one set of elements are neighbours
   const int m0 = (int)(bid % nmc) * MC, m1 = m0 + MC < a.M ? m0 + MC : a.M;
-  double* nod = smem;                          // two buffers: a slow thread still reads the other mode's
-  double* red = nod + 2 * RNS_E * RNS_EROW;
+  // staged nodal sums: written before a mode's first barrier, read between it
+  // and the second, so the next mode's writes wait for every reader
+  double* nod = smem;
+  double* red = nod + RNS_E * RNS_EROW;
   double* tab = red + (TENSOR ? 18 : 6) * RNS_SK;
   for (int i = tid; i < 126; i += RNS_THREADS) tab[i] = a.tab[i];
 
@@ -227,7 +229,6 @@ SFX_DEV void rhs_ns_tile_body(const RhsArgs& a, int tid, int64_t bid, double* sm
         }
       }
     }
-    double* nb = nod + (q & 1) * RNS_E * RNS_EROW;
     if (nslot) {
       double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
       const int64_t i6 = node + a.np * 6 * (int64_t)m, i2 = node + a.np * 2 * (int64_t)m;
@@ -266,7 +267,7 @@ SFX_DEV void rhs_ns_tile_body(const RhsArgs& a, int tid, int64_t bid, double* sm
           s[k] += a.isign * a.imp[node + a.np * k];
         }
       }
-      double2* o = reinterpret_cast<double2*>(nb + (tid / 6) * RNS_EROW + (tid % 6) * 8);
+      double2* o = reinterpret_cast<double2*>(nod + (tid / 6) * RNS_EROW + (tid % 6) * 8);
 #pragma unroll
       for (int k = 0; k < 4; ++k) o[k] = make_double2(s[2 * k], s[2 * k + 1]);
     }
@@ -280,7 +281,7 @@ SFX_DEV void rhs_ns_tile_body(const RhsArgs& a, int tid, int64_t bid, double* sm
       for (int k = 0; k < 6; ++k) f[k] = 0.0;
 #pragma unroll
       for (int n = 0; n < 6; ++n) {
-        const double2* s = reinterpret_cast<const double2*>(nb + el * RNS_EROW + n * 8);
+        const double2* s = reinterpret_cast<const double2*>(nod + el * RNS_EROW + n * 8);
         const double wn = w[n], dx = d[2 * n], dy = d[2 * n + 1];
         const double dr = fma(a11, dx, a12 * dy), dz = fma(a21, dx, a22 * dy);
 #pragma unroll
