@@ -50,8 +50,10 @@ int sfx_init(int32_t device);
  * grow-only scratch per (device, stream): calls on different streams run
  * concurrently without sharing it.  sfx_stream_release waits for the stream
  * and frees its scratch; call it before destroying a stream that ran such
- * products.  No counterpart in the reference (FFTW plans and temporary
- * arrays there are per call). */
+ * products.  With a null stream it also gives back the four page-locked chunks
+ * of 1 MB through which the host-pointer forms return results of 2 to 32 MB to
+ * pageable arrays (made again by the next such call).  No counterpart in the
+ * reference (FFTW plans and temporary arrays there are per call). */
 int sfx_stream_release(void* stream);
 
 /* ---------------------------------------------------------------------------

@@ -45,10 +45,9 @@ template <bool SPLIT> struct AdjRed { static constexpr int K = SPLIT ? 24 : 18; 
 // ms at MP = 4, 0.84 / 1.10 at 8 (both against 512 registers), 0.91 / 0.96 at 16,
 // 0.68 / 0.76 at 64 and 8.16 / 9.20 at 64 and 200,704 triangles (against 7 waves
 // with one group each, which stay at MP = 128: half tiles of one element read 56-byte
-// pieces of ybar and take 25.4 ms there against 22.6 at 200,704 triangles; a
-// wave waited 13,000 of 100,000 cycles at the barrier before the sums, three SIMDs
-// holding two waves and one holding one); split form, against 512 registers: 1.18
-// / 1.79 ms at MP = 8, 1.27 / 1.64 at 16, 1.31 / 1.68 at 32, 1.33 / 1.79 at 64.
+// pieces of ybar and take 25.4 ms there against 22.6 at 200,704 triangles); split
+// form, against 512 registers: 1.18 / 1.79 ms at MP = 8, 1.27 / 1.64 at 16, 1.31 /
+// 1.68 at 32, 1.33 / 1.79 at 64.
 template <int MP, bool SPLIT>
 constexpr bool adjoint_half() { return MP <= 64 && (!SPLIT || MP >= 8); }
 template <int MP, bool SPLIT>

@@ -69,7 +69,9 @@ SFX_DEV void batch_body(const BatchArgs& b, int tid, int wg, double2* smem) {
 }
 
 // BY_SIZE schedule: work-group bid of the grid of one grid size runs tile
-// t0 + bid with the fused kernel's own layout for that size.
+// t0 + bid on whole elements, the tiles that the schedulers cut, with that
+// size's wave count (gauss_waves); the single launch's point tiles are another
+// cut (gauss_point_tiles).
 template <int MP>
 SFX_DEV void batch_class_body(const BatchArgs& b, int32_t t0, int tid, int64_t bid, double2* smem) {
   SFX_CHECK("tile", t0 + bid, b.n_tiles);

@@ -12,8 +12,8 @@
 //                         of one problem stay on one work-group);
 //   SFX_BATCH_ROUND_ROBIN tile i to list i mod n_wg, in problem order;
 //   SFX_BATCH_BY_SIZE     one ordinary grid per grid size, launched one after
-//                         the other (each with the fused kernel's own layout
-//                         for that size; no persistent loop).
+//                         the other (each on whole elements with that size's
+//                         wave count; no persistent loop).
 //
 // The autotuner times every (policy, work-group count) candidate on the
 // caller's stream with HIP events and keeps the fastest; results are cached

@@ -89,22 +89,22 @@ SFX_DEV int lane_at(int pt, int l) { return l * Shape<MP>::PW + pt; }
 template <int MP>
 SFX_DEV int lane_partner(int pt, int l) { return lane_at<MP>(pt, (Shape<MP>::L - l) % Shape<MP>::L); }
 
-// LDS slot of (point, position) inside a wave region for exchange `ex`
-// (ex = s for the exchange between stages s and s+1, ex = 4 for the mode
-// pairing).  q = pt*MP + pos indexes the 256 slots of one signal; the low
-// four bits are XORed with a GF(2)-linear function of bits 2..7 of q.  The
-// per-exchange masks were found by exhaustive search so that every 8- and
-// 16-lane group of every access pattern hits distinct 16-byte bank groups
+// LDS slot of (point, position) inside a wave region for exchange `ex`: the one
+// between stages 2 and 3 at MP = 128 and 256 (ex = 2; the others run in registers,
+// see exchange), or the mode pairing (ex = 4).  q = pt*MP + pos indexes the 256
+// slots of one signal; the low four bits are XORed with a GF(2)-linear function
+// of bits 2..7 of q.  The masks were found by exhaustive search so that every 8-
+// and 16-lane group of every access pattern hits distinct 16-byte bank groups
 // (8-lane groups at MP = 128, ex = 4: two-way); masks on bits 2 and 3 only
-// touch bits 0 and 1, so the map is a bijection.
+// touch bits 0 and 1, so the map is a bijection.  Rows of no LDS exchange: zero.
 constexpr unsigned char SWZ[7][5][6] = {
   {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,1,2,1,0,0}},  // MP=4
-  {{0,1,4,2,1,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,1,4,2,1,0}},  // MP=8
-  {{0,0,9,4,2,1}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,9,4,2,1}},  // MP=16
-  {{0,0,0,9,4,2}, {1,0,0,9,4,2}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,1,0,9,4,2}},  // MP=32
-  {{0,0,0,0,10,4}, {1,0,0,0,10,4}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,2,0,0,10,4}},  // MP=64
-  {{0,0,0,0,0,12}, {0,2,2,0,0,12}, {1,2,2,0,0,4}, {0,0,0,0,0,0}, {0,0,0,0,0,8}},  // MP=128
-  {{0,0,0,0,0,0}, {0,0,12,4,0,0}, {2,1,12,4,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}},  // MP=256
+  {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,1,4,2,1,0}},  // MP=8
+  {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,9,4,2,1}},  // MP=16
+  {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,1,0,9,4,2}},  // MP=32
+  {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}, {0,2,0,0,10,4}},  // MP=64
+  {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {1,2,2,0,0,4}, {0,0,0,0,0,0}, {0,0,0,0,0,8}},  // MP=128
+  {{0,0,0,0,0,0}, {0,0,0,0,0,0}, {2,1,12,4,0,0}, {0,0,0,0,0,0}, {0,0,0,0,0,0}},  // MP=256
 };
 
 template <int MP>

@@ -69,13 +69,11 @@ constexpr int gauss_elems() { return 256 / MP; }
 // half the elements, 3.5 groups of points, in 256 registers per lane and at
 // most half the LDS, so that two work-groups share a CU.  The points per wave
 // are those of 7 waves with 7 groups (3.5 of 4 groups against 7 of 8 wave
-// slots), but a CU no longer stops as a whole at each barrier: a wave of the
-// 7-wave form at M = 100 spent 20,000 of 76,000 cycles waiting in the element
-// sums and 10,000 for its first chunk.  Fused right-hand side, half against whole
-// tiles: 1.23 / 1.40 ms at MP = 4 (767,000 triangles), 1.10 / 1.26 at 8, 1.14 /
-// 1.28 at 16, 1.26 / 1.42 at 32, 1.31 / 1.50 at 64, 1.49 / 1.80 at 128 (23,700);
-// u.grad c 1.25 / 1.46, 1.15 / 1.32, 1.27 / 1.47, 1.32 / 1.58, 1.48 / 1.72 and
-// 1.80 / 2.05; no slower where few work-groups run.
+// slots), but a CU no longer stops as a whole at each barrier.  Fused right-hand
+// side, half against whole tiles: 1.23 / 1.40 ms at MP = 4 (767,000 triangles), 1.10
+// / 1.26 at 8, 1.14 / 1.28 at 16, 1.26 / 1.42 at 32, 1.31 / 1.50 at 64, 1.49 / 1.80
+// at 128 (23,700); u.grad c 1.25 / 1.46, 1.15 / 1.32, 1.27 / 1.47, 1.32 / 1.58, 1.48
+// / 1.72 and 1.80 / 2.05; no slower where few work-groups run.
 template <int MP>
 constexpr bool gauss_rhs_half() { return MP <= 128; }
 template <int MP, int V>
@@ -123,7 +121,9 @@ constexpr int64_t gauss_blocks(int64_t me) {
 // (256 of them) and the point tiles would put two on some: cross-curl at MP = 8
 // 17.7 against 18.7 us with 200 whole tiles, 15.9 against 17.0 at MP = 4 and 28.7
 // against 30.0 at 128; but 15.2 against 11.5 us with 60, and 31.1 against 26.9
-// with 400.  (At 16 <= MP <= 64 the whole tiles have no instance of their own.)
+// with 400.  At 16 <= MP <= 64 three more kernels would gain less than 1.5 us (20.3
+// -> 19.7 at MP = 16 and 4,000 triangles, 23.6 -> 22.2 at 64 and 720) and are not
+// built.
 constexpr int64_t GAUSS_CUS = 256;
 template <int MP, int V>
 constexpr bool gauss_one_round() { return V == GV_CROSS_CURL && (MP < 16 || MP == 128); }
@@ -312,7 +312,7 @@ SFX_DEV T pick(const T (&v)[N], int i) {
 // slot and takes every R-th plane (several slots, every plane, where the
 // work-group has fewer threads than slots), so that its addresses advance by a
 // constant and its LDS stores have constant offsets.  The forward kernel is
-// bound by vector instruction issue (67 % of its cycles), and numbering slots,
+// bound by vector instruction issue (69 % of its cycles), and numbering slots,
 // columns and modes through one index took about 24 of them per value.
 // Measured with the interpolation below (16-byte LDS reads, only the
 // derivatives that are used) and the stores of staged outputs at constant
@@ -585,9 +585,8 @@ SFX_DEV void gauss_body(const GaussArgs& a, int tid, int64_t bid, double2* smem)
   // The first chunks' loads depend on the connectivity alone: they leave with
   // those of the tables, ahead of the first barrier and the geometry, and the
   // cross-curl's point tiles and (curl a) x b keep two chunks in flight (forward
-  // term at 200,704 triangles, M = 64, 3.81 -> 3.61 ms, of whose 59,000 cycles a
-  // wave spent 19,000 waiting for chunks; tangent at 99,856 triangles, M = 32,
-  // 2.65 -> 2.59 ms).  The element sums keep one ahead: two take 5.60 ms against
+  // term at 200,704 triangles, M = 64, 3.81 -> 3.61 ms; tangent at 99,856
+  // triangles, M = 32, 2.65 -> 2.59 ms).  The element sums keep one ahead: two take 5.60 ms against
   // 5.50 at 90,300 triangles, M = 100.
   constexpr bool EARLY = !ALL && V != GV_PAIRS;
   constexpr int NCB = (V == GV_UGRADC) ? 2 : 6;

@@ -22,9 +22,13 @@ constexpr size_t CHUNK = (size_t)1 << 20;
 // Shorter copies have too few chunks to overlap and go to hipMemcpy: 1 MB takes
 // 62 us there and 70 in the ring, 2 MB 126 and 110, 4 MB 247 and 189.
 constexpr size_t RING_MIN = 2 * CHUNK;
-// Longer ones go there too: a product with a result of 31 MB takes 3.36 ms
-// against 3.97 with hipMemcpy, but one of 58 MB took 14.4 ms against 7.4 where
-// several results were written in turn (8.4 against 9.8 at 77 MB with one).
+// Longer ones go there too.  Up to this length the ring was never slower, whole
+// calls in ms, ring / hipMemcpy: one result of 4 MB 0.46 / 0.52, of 31 MB 3.43 /
+// 3.97; two of 2.1 MB 0.69 / 0.76, of 31 MB 10.5 / 11.6; three of 2.1 MB 0.85 /
+// 0.93, of 31 MB 9.8 / 11.3; into new arrays as into old ones.  Beyond it times
+// went both ways: three of 58 MB 18.8 / 21.6, of 77 MB 24.9 / 28.3, but in an
+// earlier run one of 58 MB 14.4 against 7.4 where several results were written
+// in turn, which was not seen again and is not explained.
 constexpr size_t RING_MAX = 32 * CHUNK;
 
 struct Ring {

@@ -97,10 +97,15 @@ hipError_t launch_exact_emom(const ExactArgs& a, double* dmax, hipStream_t st);
 int64_t exact_emom_blocks(int64_t np, int lg, int K);
 #endif
 
-// Pass lists (GV_PAIRS) run as one single-pass GV_CURL_CROSS launch per
-// pass, each adding to the output, where that kernel uses seven waves of 256
-// registers (MP <= 64, measured faster than one launch of the pass list,
-// whose accumulator needs 512 registers per wave); as one launch otherwise.
+// Pass lists (GV_PAIRS) run as one single-pass GV_CURL_CROSS launch per pass,
+// each adding to the output, where that kernel runs on half tiles (point tiles at
+// MP = 4) with two waves per SIMD; as one launch, whose accumulator needs 512
+// registers per lane and one wave per SIMD, where two fields no longer fit half
+// the LDS (MP >= 128, whole tiles either way).  Passes against one launch at 50,850
+// triangles, two passes (the MHD term): 0.114 / 0.169 ms at MP = 4, 0.55 / 0.68 at
+// 16, 2.66 / 3.30 at 64, but 10.6 / 8.9 at 128.  The four passes of the MHD tangent
+// write the output once more each: 0.24 / 0.31 ms at MP = 4, but 1.24 / 1.19 at 16
+// and 6.05 / 5.48 at 64.
 inline bool pairs_as_passes(int MP) { return MP <= 64; }
 
 // Smallest supported power of two >= max(M, 4); 0 if M > 256.
