@@ -162,7 +162,7 @@ def wl_mhd(torch, args):
     rotv_bytes = 3 * npn * 6 * M * 8 + G * 6 * M * 8 + mesh_bytes
     phases = [
         Phase("rotv_mhd", lambda: NL.nl_rotv_mhd(mesh, modes, u, H, B, 1.0, work), rotv_bytes,
-              2 * b2_flops(G, M), "gauss_kernel<64,PAIRS> (2 passes)"),
+              2 * b2_flops(G, M), "gauss_half_kernel<64,CURL_CROSS> x 2"),
         # full NS RHS (rhs_ns_gauss_3x3 + rhs_3x3): rotv_v read once, V1m, ff (6 columns) and
         # P, P_inc (2 columns) read, vb written, mesh read; the element contributions
         # written and read back are re-traffic
@@ -269,15 +269,15 @@ def _exact_ops(FP, torch, npt, M, seed):
     b = 8 * M * npt
     return [
         ("heaviside", lambda: FP.FFT_HEAVISIDE_DCL(None, phi, vals, rho_out, coeff_tanh=0.05), 4 * b, 2 * f_t * npt,
-         "exact_grid_kernel<HEAVI,1> + exact_r2c_kernel"),
+         "exact_mm_kernel<HEAVI,1>"),
         ("scalar_vect_pb2", lambda: FP.FFT_SCALAR_VECT_DCL(None, mom, rho, u_out, 2), 14 * b, 7 * f_t * npt,
-         "exact_grid_kernel<SV2,4> + exact_r2c_kernel"),
+         "exact_mm_kernel<SV2,4>"),
         ("div", lambda: FP.FFT_PAR_DIV_DCL(None, c, d, q_out), 6 * b, 3 * f_t * npt,
-         "exact_grid_kernel<DIV,2> + exact_r2c_kernel"),
+         "exact_mm_kernel<DIV,2>"),
         ("squareroot", lambda: (s_io.copy_(rho_out), FP.FFT_SQUAREROOT_SCALAR(None, s_io)), 6 * b, 2 * f_t * npt,
-         "copy + exact_grid_kernel<SQRT,1> + exact_r2c_kernel"),
+         "copy + exact_mm_kernel<SQRT,1>"),
         ("tension", lambda: FP.FFT_TENSOR_DCL(None, u, g, tens, opt_tension=True), 30 * b, 15 * f_t * npt,
-         "exact_grid_kernel<TENSION,6> + exact_r2c_kernel"),
+         "exact_mm_kernel<TENSROW,4>"),
         ("max_vel", lambda: FP.FFT_MAX_VEL_DCL(None, u, V_out=vmax), 6 * b, 3 * f_t * npt,
          "exact_grid_kernel<MAXVEL,3> + exact_max_kernel"),
     ]
@@ -329,13 +329,12 @@ def wl_grid(torch, args):
         Phase("par_real", lambda: FP.FFT_PAR_REAL(None, u, planes, opt_nb_plane=N), 6 * b + 3 * r, 3 * f_t * npt,
               "exact_real_kernel x3"),
         Phase("from_real", lambda: FP.FFT_PAR_FROM_REAL(eta, back, mp), r + 2 * b, f_t * npt,
-              "exact_grid_kernel<FROMREAL,1> + exact_r2c_kernel"),
+              "exact_mm_kernel<FROMREAL,0>"),
         Phase("var_eta_prod", lambda: FP.FFT_PAR_VAR_ETA_PROD_T_DCL(None, eta, None, u, v_out), r + 12 * b,
-              6 * f_t * npt, "exact_grid_kernel<ETA3,3> + exact_r2c_kernel"),
+              6 * f_t * npt, "exact_mm_kernel<ETA3,3>"),
         Phase("compression_level_set", lambda: FP.FFT_COMPRESSION_LEVEL_SET_DCL(None, None, gphi, u, phi, c_out,
                                                                                None, 7, 1.0, 0.5, 0.01),
-              16 * b, 8 * f_t * npt, "exact_grid_kernel<MAXVEL,3> + exact_max_kernel + exact_grid_kernel<CLS,4> "
-                                     "+ exact_r2c_kernel"),
+              16 * b, 8 * f_t * npt, "exact_grid_kernel<MAXVEL,3> + exact_max_kernel + exact_mm_kernel<CLS,4>"),
         Phase("max_min_vel", lambda: FP.FFT_MAX_MIN_VEL_DCL(None, u, V_out=mm), 6 * b, 3 * f_t * npt,
               "exact_velstat_kernel<3> + exact_velstat_final_kernel"),
         Phase("check_interface", lambda: FP.FFT_CHECK_INTERFACE(None, ls, 3, interface_ok=ok), 4 * b, 2 * f_t * npt,
@@ -374,16 +373,16 @@ def wl_entropy(torch, args):
     b = 8 * M * npt
     ops = [
         ("par_entro_visc", lambda: FP.FFT_PAR_ENTRO_VISC_DCL(None, u, c, creal, None, 0.3, v6[0], c2o),
-         8 * b + 8 * N * npt, 6 * f_t * npt, "exact_grid_kernel<ENTRO,4> + exact_r2c_kernel"),
+         8 * b + 8 * N * npt, 6 * f_t * npt, "exact_mm_kernel<ENTRO,4>"),
         ("compr_entro_visc", lambda: FP.FFT_PAR_COMPR_ENTRO_VISC_DCL(None, u, g1, c, creal, None, 0.3, v6[0], c2o,
                                                                       1.5),
-         14 * b + 8 * N * npt, 11 * f_t * npt, "exact_grid_kernel<COMPR,7> + exact_r2c_kernel"),
+         14 * b + 8 * N * npt, 11 * f_t * npt, "exact_mm_kernel<COMPR,7>"),
         ("entropy_visc_grad_mom", lambda: FP.FFT_COMPUTE_ENTROPY_VISC_GRAD_MOM(None, g1, g2, g3, creal, t3, 0.2),
-         36 * b + 8 * N * npt, 18 * f_t * npt, "exact_grid_kernel<GRADMOM,9> + exact_r2c_kernel"),
+         36 * b + 8 * N * npt, 18 * f_t * npt, "exact_mm_kernel<SCALE3,3>"),
         ("entropy_visc", lambda: FP.FFT_COMPUTE_ENTROPY_VISC(None, None, u, res, g1, g2, g3, h, *v6, 1.0, lg, 0.3,
                                                              0.9, 0.8),
          48 * b + 8 * npt, 24 * f_t * npt,
-         "exact_enorm_kernel + exact_grid_kernel<EVISCV,6> + exact_grid_kernel<GRADMOM,9> + exact_r2c_kernel"),
+         "exact_enorm_kernel + exact_mm_kernel<EVISCV,6> + exact_mm_kernel<SCALE3,3>"),
         ("entropy_visc_mom", lambda: FP.FFT_COMPUTE_ENTROPY_VISC_MOM(None, None, u, mom, res, rmass, h, r1, lg, 0.6,
                                                                      0.9, opt_c2_real_out=r2),
          20 * b + 8 * npt + 16 * N * npt, 10 * f_t * npt, "exact_emom_kernel + exact_emom_out_kernel"),
@@ -433,7 +432,7 @@ def wl_tangent(torch, args):
     ab = G * 6 * M * 8 + npn * 6 * M * 8 + npn * 6 * M * 8
     phases = [
         Phase("tangent", lambda: NL.nl_tangent(mesh, modes, U, d, tout), tb,
-              2 * b2_flops(G, M), "gauss_kernel<32,PAIRS> (2 passes)"),
+              2 * b2_flops(G, M), "gauss_half_kernel<32,CURL_CROSS> x 2"),
         Phase("adjoint", lambda: NL.nl_adjoint(mesh, modes, U, ybar, dbar, work), ab,
               2 * b2_flops(G, M), "adjoint_kernel<32> + adjoint_gather_kernel",
               overhead=2 * (6 * m.me * 6 * M * 8)),
@@ -468,7 +467,7 @@ def wl_batch(torch, args):
     b.autotune(reps=2)
     b.capture()
     info = b.info()
-    phases = [Phase("batch", b.run, byts, flops, "batch_kernel (persistent, hipGraph replay)")]
+    phases = [Phase("batch", b.run, byts, flops, "the tuned schedule's kernels, one hipGraph replay")]
     cfg = {"workload": "32 independent (curl u) x u problems, 2k-50k triangles, m_max in {4..128}, "
                        "one persistent launch replayed from a hipGraph",
            "problems": 32, "triangles": int(sum(it[0].me for it in items)), "schedule": info,
