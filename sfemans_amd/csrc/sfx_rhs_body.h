@@ -159,9 +159,9 @@ inline int64_t rns_blocks(int64_t me, int M, int MC) {
 // the gather, without the tensor, one thread per (element, mode) / 8 modes / 2
 // modes: 26.5 / 28.5 / 14.9 us at 400 triangles, M = 8 (13 work-groups of 8), 107
 // / 114 / 104 at M = 128 (208), 62.8 / 57.9 / 52.0 at 3,192, M = 24 (300), but 65.6
-// / 65.8 at M = 32 (400) with 8 / 2 modes; with the tensor 67.8 / 61.5 (300) and 76.1
-// / 78.7 (400).
-constexpr int RNS_FEW = 2, RNS_FULL = 384;
+// / 65.8 at M = 32 (400) with 8 / 2 modes; with the tensor 67.8 / 61.5 (300), 77.3
+// / 79.1 at 6,084, M = 15 (382) and 76.1 / 78.7 (400).
+constexpr int RNS_FEW = 2, RNS_FULL = 320;
 inline int rns_modes(int64_t me, int M) { return rns_blocks(me, M, RNS_MC) < RNS_FULL ? RNS_FEW : RNS_MC; }
 
 template <bool TENSOR, int MC>

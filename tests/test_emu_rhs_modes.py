@@ -9,8 +9,8 @@ import pytest
 from tests import emu_runner
 
 
-# (triangles, modes): 13 work-groups of eight modes, 208, 383; 384, and the sizes of a production run
-@pytest.mark.parametrize("me,M,modes", [(400, 8, 2), (400, 128, 2), (32 * 383, 8, 2), (32 * 384, 8, 8), (102720, 48, 8),
+# (triangles, modes): 13 work-groups of eight modes, 208, 319; 320, and the sizes of a production run
+@pytest.mark.parametrize("me,M,modes", [(400, 8, 2), (400, 128, 2), (32 * 319, 8, 2), (32 * 320, 8, 8), (102720, 48, 8),
                                         (200704, 1, 8), (10**7, 256, 8)])
 def test_work_groups_fill_the_chip(me, M, modes):
     L = ctypes.CDLL(emu_runner.build_emulator())
