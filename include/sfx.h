@@ -125,7 +125,8 @@ int sfx_fft_tensor_dcl_dev(const double* V1_in, const double* V2_in, double* V_o
  * one with each (m_max_c, m_max_pad), whose tables are built at their first
  * use.  Calls that run without the scratch (on the matrix cores) reserve it
  * all the same, on any stream but the null stream and where the memory is
- * there, so any of these products serves as that call.
+ * there, so any of these products serves as that call; a smaller scratch that
+ * captured calls may hold stays beside it.
  * sfx_stream_release frees a stream's scratch.
  * The host-pointer forms stage their arrays in per-device buffers: call
  * them from one host thread at a time per device.

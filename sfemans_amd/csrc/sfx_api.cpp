@@ -105,7 +105,12 @@ int staging(int slot, size_t bytes, void** out) {
 // calls may reuse one buffer; calls on two streams get two buffers.  A buffer
 // is replaced only after its stream has drained (the kernels queued before
 // may still read the old one).
-static std::map<std::pair<int, uintptr_t>, Staging> g_stream_scratch;
+struct StreamScratch : Staging {
+  bool used[N_STAGING] = {false};   // handed out: a captured graph may hold it
+  std::vector<void*> kept;          // buffers replaced by reservations, given back with the stream's scratch
+  size_t kept_bytes = 0;
+};
+static std::map<std::pair<int, uintptr_t>, StreamScratch> g_stream_scratch;
 
 int stream_scratch(int slot, size_t bytes, hipStream_t st, void** out) {
   if (slot < 0 || slot >= N_STAGING) return fail(SFX_ERR_ARG, "scratch slot %d out of range", slot);
@@ -113,7 +118,7 @@ int stream_scratch(int slot, size_t bytes, hipStream_t st, void** out) {
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
   std::lock_guard<std::mutex> lk(g_mu);
-  Staging& s = g_stream_scratch[std::make_pair(dev, (uintptr_t)st)];
+  StreamScratch& s = g_stream_scratch[std::make_pair(dev, (uintptr_t)st)];
   if (s.n[slot] < bytes) {
     if (s.p[slot]) {
       if ((e = hipStreamSynchronize(st)) != hipSuccess) return hip_fail(e, "scratch: hipStreamSynchronize");
@@ -125,6 +130,7 @@ int stream_scratch(int slot, size_t bytes, hipStream_t st, void** out) {
     if (e != hipSuccess) return fail(SFX_ERR_NOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
     s.n[slot] = bytes;
   }
+  s.used[slot] = true;
   *out = s.p[slot];
   return SFX_OK;
 }
@@ -135,13 +141,18 @@ int stream_scratch(int slot, size_t bytes, hipStream_t st, void** out) {
 // the memory cannot be had the slot stays as it is, and only a call that uses
 // it is refused.  Nothing is done for a stream under capture, nor for the null
 // stream, which cannot be captured; other streams' captures are not disturbed
-// (relaxed mode).
+// (relaxed mode).  A smaller buffer that calls have used is kept beside the new
+// one, since a graph captured from them writes to it; kept buffers together are
+// no larger than the new one, or the slot stays as it is.
 void stream_scratch_reserve(int slot, size_t bytes, hipStream_t st) {
   int dev = 0;
   if (!st || slot < 0 || slot >= N_STAGING || hipGetDevice(&dev) != hipSuccess) return;
   std::lock_guard<std::mutex> lk(g_mu);
-  Staging& s = g_stream_scratch[std::make_pair(dev, (uintptr_t)st)];
+  StreamScratch& s = g_stream_scratch[std::make_pair(dev, (uintptr_t)st)];
   if (s.n[slot] >= bytes) return;
+  const bool keep = s.p[slot] && s.used[slot];
+  if (keep && s.kept_bytes + s.n[slot] > bytes) return;
+  if (keep) s.kept.reserve(s.kept.size() + 1);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   hipError_t e = hipStreamIsCapturing(st, &cap);
@@ -149,12 +160,16 @@ void stream_scratch_reserve(int slot, size_t bytes, hipStream_t st) {
       (e = hipThreadExchangeStreamCaptureMode(&mode)) == hipSuccess) {
     void* p = nullptr;
     e = hipMalloc(&p, bytes);
-    if (e == hipSuccess && s.p[slot] && (e = hipStreamSynchronize(st)) == hipSuccess) (void)hipFree(s.p[slot]);
     if (e == hipSuccess) {
+      if (keep) {
+        s.kept.push_back(s.p[slot]);
+        s.kept_bytes += s.n[slot];
+      } else if (s.p[slot]) {
+        (void)hipFree(s.p[slot]);   // reserved only: no queued work reads it
+      }
       s.p[slot] = p;
       s.n[slot] = bytes;
-    } else if (p) {
-      (void)hipFree(p);
+      s.used[slot] = false;
     }
     (void)hipThreadExchangeStreamCaptureMode(&mode);
   }
@@ -171,6 +186,7 @@ int release_stream_scratch(hipStream_t st) {
   if ((e = hipStreamSynchronize(st)) != hipSuccess) return hip_fail(e, "scratch release: hipStreamSynchronize");
   for (int i = 0; i < N_STAGING; ++i)
     if (it->second.p[i]) (void)hipFree(it->second.p[i]);
+  for (void* p : it->second.kept) (void)hipFree(p);
   g_stream_scratch.erase(it);
   return SFX_OK;
 }

@@ -30,6 +30,11 @@ def test_in_place_call_captured_after_a_matrix_core_warm_up(npt, M):
         x = FP.fortran_tensor(np.zeros((npt, 6, M))).copy_(v)
         want.append(FP.FFT_SCALAR_VECT_DCL(None, x, sd, x, 2))
     got, out = new((npt, 6, M)), new((npt, 6, M))
+    big = []                                                 # larger calls, on the matrix cores
+    for n in (6000, 9000):
+        x, y = torch.ones((32, 6, n), dtype=torch.float64, device="cuda"), torch.zeros((32, 2, n), dtype=torch.float64, device="cuda")
+        y[0, 0] = 2.0
+        big.append((x.permute(2, 1, 0), y.permute(2, 1, 0), new((n, 6, 32))))
     torch.cuda.synchronize()
     st = torch.cuda.Stream()
     with torch.cuda.stream(st):
@@ -39,6 +44,9 @@ def test_in_place_call_captured_after_a_matrix_core_warm_up(npt, M):
     with torch.cuda.graph(g, stream=st):
         FP.FFT_SCALAR_VECT_DCL(None, got, sd, got, 2)
     for i in (0, 1, 0):
+        with torch.cuda.stream(st):                          # they reserve more scratch; the graph's stays
+            FP.FFT_SCALAR_VECT_DCL(None, *big[i], 2)
+        st.synchronize()
         got.copy_(Vd[i])
         torch.cuda.synchronize()
         g.replay()

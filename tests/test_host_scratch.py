@@ -90,3 +90,27 @@ def test_null_stream_and_release(L):
     assert sv2(L, O, 5000, 16, stream=None) == 0 and L.fake_used() == tables
     assert sv2(L, O, 5000, 16) == 0 and L.fake_used() == tables + 2 * 3 * 24 * 5000 * 8
     assert L.sfx_stream_release(STREAM) == 0 and L.fake_used() == tables
+
+
+def test_a_captured_scratch_outlives_larger_matrix_core_calls(L):
+    # a graph holds the scratch of an in-place call; larger calls on the matrix cores reserve more, and leave it
+    assert sv2(L, A, 3000, 16) == 0
+    L.fake_reset_counts()
+    assert sv2(L, O, 5000, 16) == 0 and routes(L) == (1, 0)
+    assert L.fake_count(b"free") == 0
+    L.fake_capture(STREAM, 1)                              # and a larger in-place call can be captured after it
+    rc = sv2(L, A, 5000, 16)
+    broken = L.fake_capture_broken()
+    L.fake_capture(None, 0)
+    assert rc == 0 and not broken and L.fake_count(b"free") == 0
+
+
+def test_scratch_is_bounded_and_given_back(L):
+    assert sv2(L, O, 100, 16, stream=None) == 0
+    tables = L.fake_used()
+    for n in range(1000, 9000, 500):                       # growing calls on both kinds of kernels in turn
+        assert sv2(L, A, n, 16) == 0 and sv2(L, O, n + 250, 16) == 0
+        assert L.fake_used() - tables <= 2 * (2 * 3 * 24 * (n + 250) * 8)
+    for n in range(10000, 20000, 1000):                    # on the matrix cores alone: one buffer
+        assert sv2(L, O, n, 16) == 0
+    assert L.sfx_stream_release(STREAM) == 0 and L.fake_used() == tables
